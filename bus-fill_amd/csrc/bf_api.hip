@@ -150,10 +150,14 @@ bf_status check_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uin
     return BF_OK;
 }
 
+// The prefill tile kernel (more than 128 rows in one launch): chosen by the
+// automatic plan only, so not a bf_algo a caller can name.
+constexpr int kAlgoTile = 100;
+
 // One launch of a bf_gemm call: a slice of batch rows and its kernel.
 struct Planned {
     bf::GemmArgs g;
-    bf_algo use;
+    int use;                              // a bf_algo, or kAlgoTile
 };
 
 // The launches a call makes, each checked against its kernel's limits before
@@ -184,6 +188,13 @@ bf_status plan_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uint
         g.K = K;
         return g;
     };
+    if (algo == BF_ALGO_AUTO && M > kMaxMPerLaunch) {
+        const bf::GemmArgs g = args(0, M);
+        if (fast_eligible(g) && bf::tile_supports(g)) {
+            out.push_back(Planned{g, kAlgoTile});
+            return BF_OK;
+        }
+    }
     if (algo == BF_ALGO_AUTO && M > kSplitMaxM) {
         bf::GemmArgs probe = args(0, M < kMaxMPerLaunch ? M : kMaxMPerLaunch);
         dense_slices = fast_eligible(probe) && bf::dense_supports(probe);
@@ -247,6 +258,7 @@ bf_status plan_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uint
 size_t scratch_need(const Planned& l) {
     if (l.use == BF_ALGO_SPLIT) return bf::split_scratch_bytes(l.g);
     if (l.use == BF_ALGO_DENSE) return bf::dense_scratch_bytes(l.g);
+    if (l.use == kAlgoTile) return bf::tile_scratch_bytes(l.g);
     return 0;
 }
 
@@ -254,10 +266,16 @@ size_t scratch_need(const Planned& l) {
 bf::WsNeed ws_need(const Planned& l) {
     if (l.use == BF_ALGO_SPLIT) return bf::split_ws_need(l.g);
     if (l.use == BF_ALGO_DENSE) return bf::dense_ws_need(l.g);
+    if (l.use == kAlgoTile) return bf::tile_ws_need(l.g);
     return bf::WsNeed{};
 }
 
-const char* kernel_name(bf_algo a) { return a == BF_ALGO_SPLIT ? "K-split" : a == BF_ALGO_DENSE ? "dense" : "other"; }
+const char* kernel_name(int a) {
+    return a == BF_ALGO_SPLIT ? "K-split" : a == BF_ALGO_DENSE ? "dense" : a == kAlgoTile ? "tile" : "other";
+}
+
+// Launches that share the stream's workspace (or a caller's) with others.
+bool uses_workspace(int a) { return a == BF_ALGO_SPLIT || a == BF_ALGO_DENSE || a == kAlgoTile; }
 
 // Before anything is enqueued: a caller's buffer must hold every launch's
 // need (the launches run in stream order, so they share it); otherwise the
@@ -289,9 +307,10 @@ bf_status launch_planned(const Planned& l, const bf::Scratch* scratch, hipStream
         case BF_ALGO_SPLIT: e = bf::gemm_split(l.g, scratch, hs); break;
         case BF_ALGO_DENSE: e = bf::gemm_dense(l.g, scratch, hs); break;
         case BF_ALGO_LDS: e = bf::gemm_lds(l.g, hs); break;
+        case kAlgoTile: e = bf::gemm_tile(l.g, scratch, hs); break;
         default: e = bf::gemm_simple(l.g, hs); break;
     }
-    return l.use == BF_ALGO_SPLIT || l.use == BF_ALGO_DENSE ? from_split(e, "kernel launch") : from_hip(e, "kernel launch");
+    return uses_workspace(l.use) ? from_split(e, "kernel launch") : from_hip(e, "kernel launch");
 }
 
 // scratch: the caller's workspace (bf_gemm_ws, bf_gemm_noalloc) or nullptr
@@ -311,7 +330,7 @@ bf_status run_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uint1
     // calls on the LDS-staged and other single-launch kernels share nothing
     // between launches: no lock on the batch 1-8 path
     bool shares = scratch != nullptr;
-    for (const Planned& l : ls) shares = shares || l.use == BF_ALGO_SPLIT || l.use == BF_ALGO_DENSE;
+    for (const Planned& l : ls) shares = shares || uses_workspace(l.use);
     std::unique_lock<std::recursive_mutex> held;
     if (shares) held = stream_lock(stream);
     st = secure_workspace(ls, scratch, hs, who, holder);

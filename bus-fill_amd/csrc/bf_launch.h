@@ -18,7 +18,7 @@ struct GemmArgs {
     void* C;                   // [M][ldc] fp32 or fp16
     int ldc;
     int out_f16;
-    int M, N, K;               // M <= 128 per launch (the front end slices larger M)
+    int M, N, K;               // M <= 128 per launch (the front end slices larger M), but in gemm_tile
     int a_f32 = 0;             // A is fp32 rows, lda in floats (rounded to fp16 as loaded: lds_f32_supports)
 };
 
@@ -109,6 +109,13 @@ hipError_t gemm_dense_batched(const GemmArgs* gs, int n, const Scratch* scratch,
 bool dense_batched_supports(const GemmArgs* gs, int n);
 size_t dense_batched_scratch_bytes(const GemmArgs* gs, int n);
 WsNeed dense_batched_ws_need(const GemmArgs* gs, int n);
+// The tile kernel (more than 128 batch rows in one launch; g.M unbounded):
+// workspace for the K ranges of the tiles that do not fill a round of
+// workgroups, summed by a second launch.
+hipError_t gemm_tile(const GemmArgs& g, const Scratch* scratch, hipStream_t st);
+bool tile_supports(const GemmArgs& g);
+size_t tile_scratch_bytes(const GemmArgs& g);
+WsNeed tile_ws_need(const GemmArgs& g);
 
 hipError_t dequant_f16(int qtype, const uint8_t* W, const uint8_t* Waux, uint16_t* out,
                        int N, int K, hipStream_t st);
