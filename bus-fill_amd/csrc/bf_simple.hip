@@ -6,7 +6,7 @@
 // (q - 8) * d and (d*sc)*q are exact products in fp32, so fused and unfused
 // evaluation agree and the only rounding is the final v_cvt_f16_f32 (RNE,
 // fp16 denormals preserved).
-#include "bf_device.h"
+#include "bf_formats.h"
 #include "bf_launch.h"
 
 namespace bf {
@@ -43,7 +43,8 @@ __device__ __forceinline__ float elem_f32(int qt, const uint8_t* W, const uint8_
     return __builtin_fmaf(d * (float)sc, (float)q, -(dmin * (float)m));
 }
 
-// One thread per 32-element group (a Q4_0 block or a Q4_K sub-block).
+// One thread per 32-element group (a Q4_0 block or a Q4_K sub-block): weights
+// or output off their 16-byte boundaries.
 __global__ __launch_bounds__(256) void k_dequant_f16(int qt, const uint8_t* __restrict__ W,
                                                      const uint8_t* __restrict__ Waux,
                                                      uint16_t* __restrict__ out, int N, int K) {
@@ -61,9 +62,80 @@ __global__ __launch_bounds__(256) void k_dequant_f16(int qt, const uint8_t* __re
     }
 }
 
+// Wide form: eight weights per thread, the GEMMs' decode, and a
+// 16-byte store past the caches (nt), so that a wave's store is 1 KB in one
+// piece.  Rows follow each other without gaps in every format and in the
+// output, so a thread's bytes and results follow from its number alone; both
+// nibbles' threads read the same code bytes.  Bound by HBM: 17408 x 5120 reads
+// 50 MB and writes 178 MB; Q4_K 918 -> 32 us (7.1 TB/s).  Two
+// stores of 16 bytes per thread, both nibbles of its bytes: 48 us (Q4_K) and
+// 89 us (Q4_0); plain stores 49-59 us; 2 / 4 / 8 such units per thread 33 / 34 /
+// 35 us.
+template <int QT> struct DqUnit { uint32_t x, y; u4 hdr; };
+
+struct __attribute__((packed, aligned(2))) U2a2 { uint32_t x, y; };
+
+template <int QT>
+__device__ __forceinline__ void dq_load(DqUnit<QT>& u, const uint8_t* __restrict__ W, const uint8_t* __restrict__ Waux,
+                                        int64_t t) {
+    if constexpr (QT == QT_Q4_K) {                     // 32 units per super-block: chunk, nibble, eight bytes
+        const uint8_t* p = W + (t >> 5) * 144;
+        const int i = (int)t & 31;
+        u.hdr = *(const u4*)p;
+        const uint2 v = *(const uint2*)(p + 16 + 32 * (i >> 3) + 8 * (i & 3));
+        u.x = v.x;
+        u.y = v.y;
+    } else if constexpr (QT == QT_PLANES) {            // four units per scale
+        u.x = *(const uint32_t*)(W + 4 * t);
+        u.hdr.x = *(const uint16_t*)(Waux + 2 * (t >> 2));
+    } else {                                           // four units per block: bytes 8 (t % 2) .. of nibble t / 2 % 2
+        const uint8_t* p = W + (t >> 2) * 18;
+        u.hdr.x = *(const uint16_t*)p;
+        const U2a2 v = *(const U2a2*)(p + 2 + 8 * ((int)t & 1));
+        u.x = v.x;
+        u.y = v.y;
+    }
+}
+
+template <int QT>
+__device__ __forceinline__ void dq_store(const Magic& mg, const DqUnit<QT>& u, uint16_t* __restrict__ out, int64_t t) {
+    if constexpr (QT == QT_Q4_K) {
+        Raw<QT_Q4_K> raw;
+        raw.hdr = u.hdr;
+        const Scl<QT_Q4_K> s = scales(raw, ((int)t & 31) >> 3);
+        const bool hi = (int)t & 4;                    // sb is d sc 2^20, for codes left in the high nibble
+        const int sh = hi ? 4 : 0;
+        __builtin_nontemporal_store(decode8_mix<false>(u.x >> sh, u.y >> sh, hi ? s.sb * 16.0f : s.sa, hi ? s.cb : s.ca),
+                                    (h8*)(out + 8 * t));
+    } else if constexpr (QT == QT_PLANES) {
+        __builtin_nontemporal_store(decode8_planes(mg, u.x, splat(u.hdr.x)), (h8*)(out + 8 * t));
+    } else {
+        const int sh = 2 * ((int)t & 2);
+        __builtin_nontemporal_store(decode8_q4_0<false>(mg, u.x >> sh, u.y >> sh, splat(u.hdr.x)), (h8*)(out + 8 * t));
+    }
+}
+
+template <int QT>
+__global__ __launch_bounds__(256) void k_dequant_f16_wide(const uint8_t* __restrict__ W,
+                                                          const uint8_t* __restrict__ Waux,
+                                                          uint16_t* __restrict__ out, int64_t units) {
+    const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (t >= units) return;
+    DqUnit<QT> u;
+    dq_load<QT>(u, W, Waux, t);
+    dq_store<QT>(make_magic(), u, out, t);
+}
+
 hipError_t dequant_f16(int qtype, const uint8_t* W, const uint8_t* Waux, uint16_t* out, int N, int K,
                        hipStream_t st) {
-    const int64_t groups = (int64_t)N * (K >> 5);
+    const int64_t groups = (int64_t)N * (K >> 5), units = 4 * groups;
+    const int64_t wide = (units + 255) / 256;
+    if ((((uintptr_t)out | (qtype == QT_Q4_0 ? 0 : (uintptr_t)W)) & 15) == 0 && wide < (int64_t(1) << 31)) {
+        auto k = qtype == QT_Q4_K ? k_dequant_f16_wide<QT_Q4_K>
+                 : qtype == QT_PLANES ? k_dequant_f16_wide<QT_PLANES> : k_dequant_f16_wide<QT_Q4_0>;
+        hipLaunchKernelGGL(k, dim3((unsigned)wide), dim3(256), 0, st, W, Waux, out, units);
+        return hipGetLastError();
+    }
     int64_t blocks = (groups + 255) / 256;
     if (blocks > 8192) blocks = 8192;
     hipLaunchKernelGGL(k_dequant_f16, dim3((unsigned)blocks), dim3(256), 0, st, qtype, W, Waux, out, N, K);
