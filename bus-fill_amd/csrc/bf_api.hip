@@ -150,14 +150,16 @@ bf_status check_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uin
     return BF_OK;
 }
 
-// The prefill tile kernel (more than 128 rows in one launch): chosen by the
-// automatic plan only, so not a bf_algo a caller can name.
+// Kernels of the automatic plan only, so not a bf_algo a caller can name.  The
+// prefill tile kernel: more than 128 rows in one launch.
 constexpr int kAlgoTile = 100;
+// The block-wise kernel: Q4_0 formats off the fast kernels' grid, any batch.
+constexpr int kAlgoBlock = 101;
 
 // One launch of a bf_gemm call: a slice of batch rows and its kernel.
 struct Planned {
     bf::GemmArgs g;
-    int use;                              // a bf_algo, or kAlgoTile
+    int use;                              // a bf_algo, kAlgoTile or kAlgoBlock
 };
 
 // The launches a call makes, each checked against its kernel's limits before
@@ -192,6 +194,13 @@ bf_status plan_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uint
         const bf::GemmArgs g = args(0, M);
         if (fast_eligible(g) && bf::tile_supports(g)) {
             out.push_back(Planned{g, kAlgoTile});
+            return BF_OK;
+        }
+    }
+    if (algo == BF_ALGO_AUTO) {
+        const bf::GemmArgs g = args(0, M);             // (every slice of rows is as aligned as the first)
+        if (!fast_eligible(g) && bf::block_supports(g)) {
+            out.push_back(Planned{g, kAlgoBlock});
             return BF_OK;
         }
     }
@@ -308,6 +317,7 @@ bf_status launch_planned(const Planned& l, const bf::Scratch* scratch, hipStream
         case BF_ALGO_DENSE: e = bf::gemm_dense(l.g, scratch, hs); break;
         case BF_ALGO_LDS: e = bf::gemm_lds(l.g, hs); break;
         case kAlgoTile: e = bf::gemm_tile(l.g, scratch, hs); break;
+        case kAlgoBlock: e = bf::gemm_block(l.g, hs); break;
         default: e = bf::gemm_simple(l.g, hs); break;
     }
     return uses_workspace(l.use) ? from_split(e, "kernel launch") : from_hip(e, "kernel launch");

@@ -18,7 +18,7 @@ struct GemmArgs {
     void* C;                   // [M][ldc] fp32 or fp16
     int ldc;
     int out_f16;
-    int M, N, K;               // M <= 128 per launch (the front end slices larger M), but in gemm_tile
+    int M, N, K;               // M <= 128 per launch (the front end slices larger M), but in gemm_tile and gemm_block
     int a_f32 = 0;             // A is fp32 rows, lda in floats (rounded to fp16 as loaded: lds_f32_supports)
 };
 
@@ -116,6 +116,10 @@ hipError_t gemm_tile(const GemmArgs& g, const Scratch* scratch, hipStream_t st);
 bool tile_supports(const GemmArgs& g);
 size_t tile_scratch_bytes(const GemmArgs& g);
 WsNeed tile_ws_need(const GemmArgs& g);
+
+// The block-wise kernel (Q4_0 formats; any K % 32 == 0, alignment and batch).
+hipError_t gemm_block(const GemmArgs& g, hipStream_t st);
+bool block_supports(const GemmArgs& g);
 
 hipError_t dequant_f16(int qtype, const uint8_t* W, const uint8_t* Waux, uint16_t* out,
                        int N, int K, hipStream_t st);

@@ -1,0 +1,70 @@
+"""The block-wise GEMM (bf_gemm for Q4_0 formats with K % 256 != 0 or operands
+off their 16-byte boundaries) against the one-thread-per-output kernel on the
+same inputs (run on an MI355X).
+
+Neither rounds a weight and both accumulate in fp32, over at most K + 8 terms
+in orders of their own, so the two differ by at most 2 (K + 8) * 2^-24 *
+sum_k |a w| (fp16 outputs: plus the rounding)."""
+import numpy as np
+import pytest
+import torch
+
+import busfill as bf
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+QTS = [O.Q4_0_PLANES, O.Q4_0]
+QT_NAME = {O.Q4_0_PLANES: "planes", O.Q4_0: "q4_0"}
+
+
+def to_dev(a, shift=0):
+    """On the device, `shift` elements into a buffer of its own."""
+    t = torch.from_numpy(np.ascontiguousarray(a).view(np.int16 if a.dtype == np.uint16 else a.dtype))
+    buf = torch.zeros(t.numel() + 16, dtype=t.dtype, device="cuda")
+    buf[shift:shift + t.numel()] = t.reshape(-1).cuda()
+    return buf[shift:]
+
+
+def run(qt, w, A, M, N, K, *, algo=bf.ALGO_AUTO, a_shift=0, w_shift=0, pad=0, otype=bf.OUT_F32):
+    lda = K + pad
+    Ax = np.zeros((M, lda), np.uint16)
+    Ax[:, :K] = A
+    C = torch.full((M, N + pad), -7.0, device="cuda", dtype=torch.float32 if otype == bf.OUT_F32 else torch.float16)
+    bf.gemm(qt, to_dev(w.W, w_shift), to_dev(w.W_aux, w_shift // 2) if w.W_aux is not None else None,
+            to_dev(Ax, a_shift), C, M, N, K, lda=lda, ldc=N + pad, algo=algo, otype=otype)
+    assert (C[:, N:] == -7.0).all()
+    return C[:, :N].cpu().numpy()
+
+
+@pytest.mark.parametrize("qt", QTS, ids=lambda q: QT_NAME[q])
+@pytest.mark.parametrize("M,N,K,a_shift,w_shift,pad", [
+    (1, 1, 32, 0, 0, 0), (16, 15, 96, 0, 0, 0), (17, 33, 288, 0, 0, 3), (48, 300, 160, 1, 0, 0), (64, 17, 1184, 0, 0, 5),
+    (65, 100, 2336, 3, 2, 1), (1, 4900, 416, 0, 0, 0), (129, 1700, 96, 0, 0, 0), (5, 70, 512, 1, 0, 1),
+    (140, 64, 1024, 0, 2, 0)])
+def test_block_matches_simple(qt, M, N, K, a_shift, w_shift, pad):
+    w = O.gen_weights(qt, N, K, seed=N + K)
+    A = O.gen_act(M, K, seed=M + K)
+    kw = dict(a_shift=a_shift, w_shift=w_shift, pad=pad)
+    C = run(qt, w, A, M, N, K, **kw)
+    D = run(qt, w, A, M, N, K, algo=bf.ALGO_SIMPLE, **kw)
+    mag = np.abs(O.f16_bits_to_f32(A)).astype(np.float64) @ np.abs(O.dequant_f32(w)).astype(np.float64).T
+    assert (np.abs(C.astype(np.float64) - D) <= 2 * (K + 8) * 2.0 ** -24 * mag).all()
+    assert (run(qt, w, A, M, N, K, **kw) == C).all()
+    assert (run(qt, w, A, M, N, K, otype=bf.OUT_F16, **kw) == C.astype(np.float16)).all()
+
+
+@pytest.mark.parametrize("qt", QTS, ids=lambda q: QT_NAME[q])
+def test_block_non_finite_rows(qt):
+    """An infinite or NaN activation, and an infinite scale, reach the same
+    outputs as in the one-thread-per-output kernel and no others."""
+    M, N, K = 20, 40, 352
+    w = O.gen_weights(qt, N, K, seed=9)
+    scales = w.W_aux if qt == O.Q4_0_PLANES else w.W.reshape(N, K // 32, 18)[:, :, :2].view(np.uint16)[..., 0]
+    scales[3, 5] = 0x7C00
+    A = O.gen_act(M, K, seed=10)
+    A[2, 7], A[11, 100], A[19, 351] = 0x7C00, 0x7E00, 0xFC00
+    C, D = run(qt, w, A, M, N, K), run(qt, w, A, M, N, K, algo=bf.ALGO_SIMPLE)
+    assert (np.isfinite(C) == np.isfinite(D)).all()
+    assert not np.isfinite(C[[2, 11, 19]]).any() and not np.isfinite(C[:, 3]).any()
+    assert np.isfinite(np.delete(np.delete(C, [2, 11, 19], 0), 3, 1)).all()
