@@ -522,7 +522,7 @@ struct GgmlCall {
     int64_t K = 0, N = 0, M = 0, ne2 = 1, ne3 = 1, r2 = 1, r3 = 1;
     bool stage = false;            // src1 goes through the fp16 staging buffer
     size_t stage_bytes = 0;
-    bool fused = false;            // one fp32 row on the batch-1 LDS kernel, rounded as it loads (fg)
+    bool fused = false;            // a few fp32 rows on the LDS kernel, rounded as it loads them (fg)
     bf::GemmArgs fg;
 };
 
@@ -588,11 +588,11 @@ bf_status check_ggml(const bf_ggml_tensor* s0, const bf_ggml_tensor* s1, const b
                 (((uintptr_t)s1->data | s1->nb[1] | s1->nb[2] | s1->nb[3]) & 15) == 0 &&
                 s1->nb[1] / 2 >= (uint64_t)c.K && s1->nb[1] / 2 <= INT32_MAX);
     c.stage_bytes = c.stage ? align256((size_t)(c.M * c.ne2 * c.ne3) * (size_t)c.K * 2) : 0;
-    // One or two fp32 rows (decode steps) where bf_gemm would run the LDS
-    // kernel on their fp16 copy in a form whose compute waves load all of A:
-    // that kernel rounds the rows as it loads them (the same rounding, so the
+    // Up to eight fp32 rows (decode steps) where bf_gemm would run the LDS
+    // kernel on their fp16 copy with all of A in LDS: that kernel rounds the
+    // rows as its compute waves load them (the same rounding and sums, so the
     // same bits), and no staging launch runs.
-    if (s1->type == BF_GGML_F32 && c.M <= 2 && c.ne2 * c.ne3 == 1 && s1->nb[0] == 4 &&
+    if (s1->type == BF_GGML_F32 && c.M <= 8 && c.ne2 * c.ne3 == 1 && s1->nb[0] == 4 &&
         (((uintptr_t)s1->data | s1->nb[1]) & 15) == 0 && s1->nb[1] / 4 >= (uint64_t)c.K &&
         s1->nb[1] / 4 <= INT32_MAX) {
         const uint16_t* const fake = (const uint16_t*)(uintptr_t)0x100000;   // aligned fp16 rows (the plan's view)

@@ -90,6 +90,8 @@ namespace {
 // (lda in floats), rounded to fp16 as the compute waves load them.  EA (plans
 // whose steps all have a slot of their own, no step ring): each loader issues
 // the first group's step before the rest of its setup.
+constexpr int kAfBatch = 2;              // activation instructions of a wave in flight (AF)
+
 template <int QT, int G, int MT, int NC, int NL, bool BD, bool RG, bool AC, bool SW = false, bool DEP = false,
           bool CO = false, bool AF = false, bool EA = false>
 __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* __restrict__ W,
@@ -440,24 +442,49 @@ __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* _
             clear_flags_and_meet();
             wait_dep();
         }
-        for (int f = cw; f < nsteps * IA; f += NC) {
-            const int sg = f / IA, i = f - sg * IA;
+        auto piece = [&](int f, int& sg, int& i, bool& on) {
+            sg = f / IA;
+            i = f - sg * IA;
             const uint32_t P = 64u * i + lane;
             const uint32_t m = P / (33u * G), rem = P - 33u * G * m, gg = rem / 33u, c = rem - 33u * gg;
-            const int64_t elem = (int64_t)min((int)m, M - 1) * lda + 256 * (G * sg + gg) + 8 * min((int)c, 31);
+            on = P < (uint32_t)PA && c < 32;
+            return (int64_t)min((int)m, M - 1) * lda + 256 * (G * sg + gg) + 8 * min((int)c, 31);
+        };
+        if constexpr (AF) {
+            // fp32 rows through registers: kAfBatch instructions' loads in flight
+            // together (5120^2 Q4_K at batch 2 / 8: 7.1 / 10.1 us with two, 7.6 /
+            // 10.1 with four, 8.7 / 10.1 with eight)
+            for (int f0 = cw; f0 < nsteps * IA; f0 += kAfBatch * NC) {
+                f4 v[kAfBatch][2];
+                int sg[kAfBatch], i[kAfBatch];
+                bool on[kAfBatch];
+#pragma unroll
+                for (int u = 0; u < kAfBatch; u++) {
+                    const float* src = (const float*)(const void*)A + piece(f0 + u * NC, sg[u], i[u], on[u]);
+                    on[u] = on[u] && f0 + u * NC < nsteps * IA;
+                    if (on[u]) {
+                        v[u][0] = *(const f4*)src;
+                        v[u][1] = *(const f4*)(src + 4);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kAfBatch; u++)
+                    if (on[u])
+                        *(u4*)(lds + kFlagBytes + sg[u] * seg_bytes + (i[u] << 10) + 16 * lane) =
+                            f32x8_to_f16(v[u][0], v[u][1]);
+            }
+        }
+        for (int f = cw; !AF && f < nsteps * IA; f += NC) {
+            int sg, i;
+            bool on;
+            const int64_t elem = piece(f, sg, i, on);
             const uint16_t* src = A + elem;
             if constexpr (SW && DEP) {
-                if (P < (uint32_t)PA && c < 32)
-                    *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) = swiglu_dep(elem);
+                if (on) *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) = swiglu_dep(elem);
             } else if constexpr (SW) {
-                if (P < (uint32_t)PA && c < 32)
-                    *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) = swiglu8(src, src + K);
-            } else if constexpr (AF) {
-                if (P < (uint32_t)PA && c < 32)
-                    *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) =
-                        f32x8_to_f16((const float*)(const void*)A + elem);
+                if (on) *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) = swiglu8(src, src + K);
             } else {
-                if (P < (uint32_t)PA && c < 32) dma16(src, lds0 + (uint32_t)(kFlagBytes + sg * seg_bytes + (i << 10)));
+                if (on) dma16(src, lds0 + (uint32_t)(kFlagBytes + sg * seg_bytes + (i << 10)));
             }
         }
         if constexpr (!DEP) clear_flags_and_meet();
@@ -924,9 +951,10 @@ hipError_t dispatch_lds(const GemmArgs& g, const LdsPlan& p, hipStream_t st) {
     if (g.a_f32) {
         if (p.BD) return ea ? launch_lds<QT, 4, 1, true, false, false, false, true, true>(g, p, st)
                             : launch_lds<QT, 4, 1, true, false, false, false, true>(g, p, st);
-        if (p.AC) return ea ? launch_lds<QT, 4, 1, false, false, true, false, true, true>(g, p, st)
-                            : launch_lds<QT, 4, 1, false, false, true, false, true>(g, p, st);
-        return hipErrorInvalidValue;
+        if (p.MT == 2) return ea ? launch_lds<QT, 4, 2, false, false, true, false, true, true>(g, p, st)
+                                 : launch_lds<QT, 4, 2, false, false, true, false, true>(g, p, st);
+        return ea ? launch_lds<QT, 4, 1, false, false, true, false, true, true>(g, p, st)
+                  : launch_lds<QT, 4, 1, false, false, true, false, true>(g, p, st);
     }
     if (p.BD) return ea ? launch_lds<QT, 4, 1, true, false, false, false, false, true>(g, p, st)
                         : launch_lds<QT, 4, 1, true>(g, p, st);
@@ -1178,15 +1206,25 @@ bool lds_supports(const GemmArgs& g) {
     return choose_lds(lds_shape(g), p);
 }
 
+// fp32 rows (the ggml hook): plans that keep all of A in LDS, in the form whose
+// compute waves load it.  Up to batch 8 that costs no more than the staging launch
+// the rows would otherwise take, although the loaders' way is faster for fp16
+// rows (Q4_K, us, batch 3 / 5 / 8: 5120^2 10.4 / 11.0 / 11.3 -> 7.6 / 8.8 /
+// 10.1; 17408 x 5120 16.6 / 18.5 / 19.1 -> 13.3 / 15.9 / 17.8; 3000 x 8192
+// 10.3 / 11.6 / 13.2 -> 7.8 / 9.8 / 13.3).
+bool lds_f32_plan(const GemmArgs& g, LdsPlan& p) {
+    return choose_lds(lds_shape(g), p) && (p.BD || (!p.RG && p.G == 4));
+}
+
 bool lds_f32_supports(const GemmArgs& g) {
     LdsPlan p;
     if (((uintptr_t)g.A & 15) || (g.lda & 3) || (g.qtype == QT_PLANES && ((uintptr_t)g.Waux & 15))) return false;
-    return choose_lds(lds_shape(g), p) && (p.BD || p.AC);
+    return lds_f32_plan(g, p);
 }
 
 hipError_t gemm_lds(const GemmArgs& g, hipStream_t st) {
     LdsPlan p;
-    if (!choose_lds(lds_shape(g), p)) return hipErrorInvalidValue;
+    if (!(g.a_f32 ? lds_f32_plan(g, p) : choose_lds(lds_shape(g), p))) return hipErrorInvalidValue;
     switch (g.qtype) {
         case QT_Q4_K: return dispatch_lds<QT_Q4_K>(g, p, st);
         case QT_PLANES: return dispatch_lds<QT_PLANES>(g, p, st);

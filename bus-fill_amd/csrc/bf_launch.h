@@ -34,8 +34,8 @@ hipError_t gemm_mfma(const GemmArgs& g, hipStream_t st);
 hipError_t gemm_dot2(const GemmArgs& g, hipStream_t st);
 hipError_t gemm_simple(const GemmArgs& g, hipStream_t st);
 hipError_t gemm_lds(const GemmArgs& g, hipStream_t st);
-// g with a_f32 set: the LDS kernel of bf_gemm's plan for g's shape in a form
-// whose compute waves load all of A (batch 1, and batch 2 where A fits), then
+// g with a_f32 set: the LDS kernel of bf_gemm's plan for g's shape, where that
+// keeps all of A in LDS (batch 1-8), in the form whose compute waves load A,
 // rounding the fp32 rows to fp16 as they load them.
 bool lds_f32_supports(const GemmArgs& g);
 bool lds_supports(const GemmArgs& g);
