@@ -22,11 +22,15 @@
 // latency: eight blocks in flight or 4 / 16 waves change nothing, and 4-byte
 // code loads with two 8-byte activation loads gain 10 % at M = 1 and lose
 // 15-25 % from M = 37.
+//
+// Where that takes more than a round of workgroups, k_gemm_block_staged passes
+// the activations through LDS (below).
 #include <algorithm>
 #include <type_traits>
 
 #include "bf_formats.h"
 #include "bf_launch.h"
+#include "bf_lds.h"
 
 namespace bf {
 namespace {
@@ -169,16 +173,249 @@ void k_gemm_block(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Wau
     }
 }
 
-struct BlockPlan { int MT, NT, nb; int64_t grid; };
+// The staged form: a workgroup computes 16 MT batch rows x 16 NW weight rows (a
+// wave 16 of them), K in steps of four blocks.  The activations of a step go
+// through LDS, loaded four steps ahead in 16-byte pieces along the rows, so
+// each is read once per 64 or 128 weight rows instead of 16 or 32; four lanes
+// load a weight row's four blocks whole (two loads where block by block takes
+// eight) and swap them by permlane.  NW = 4: two groups of four waves halve K.
+//
+// Measured (us per GEMM, k_gemm_block -> here, Q4_0 / planes): 5000 x 5152 at
+// M = 300 120 / 89 -> 55 / 41, M = 129 62 / 47 -> 32 / 22, M = 80 51 / 36 ->
+// 32 / 22; 3001 x 2336 at M = 300 31 / 25 -> 20 / 16; 4500 x 672 at M = 300
+// 15.9 / 13.3 -> 13.0 / 10.5.  Error against 64-bit sums 0.9e-7 .. 2.3e-7 (the
+// one-thread-per-output kernel 8e-7 .. 1.2e-6).  Bound by a wave's own chain
+// of 200-220 instructions per step: eight waves on the same rows take as long
+// as four, and halving K over two groups of waves gains where halving the rows
+// does not.  Loads under a branch drained all of them at every step (60 us).
+constexpr int kStBlocks = 4;             // blocks of a step
+constexpr int kStAhead = 4;              // steps whose loads are in flight
+
+struct __attribute__((packed, aligned(1))) B16a1 { uint32_t x, y, z, w; };
+
+// Lane (r, g) of a wave holds block b + g of its weight row: four words of
+// codes and the scale (four lanes' loads cover a row's 72 or 64 bytes).
+struct StRaw { uint32_t w[4]; uint16_t d; };
+
+template <int QT>
+__device__ __forceinline__ StRaw st_load(const uint8_t* row, const uint8_t* aux, int b) {
+    StRaw o;
+    if constexpr (QT == QT_Q4_0) {
+        const uint8_t* p = row + 18 * (int64_t)b;
+        const B16a2 v = *(const B16a2*)(p + 2);
+        o.w[0] = v.x; o.w[1] = v.y; o.w[2] = v.z; o.w[3] = v.w;
+        o.d = *(const uint16_t*)p;
+    } else {
+        const B16a1 v = *(const B16a1*)(row + 16 * (int64_t)b);
+        o.w[0] = v.x; o.w[1] = v.y; o.w[2] = v.z; o.w[3] = v.w;
+        o.d = *(const uint16_t*)(aux + 2 * (int64_t)b);
+    }
+    return o;
+}
+
+// Rows of 16 lanes: (a0 a1 a2 a3), (b0 b1 b2 b3) -> (a0 a1 b0 b1), (a2 a3 b2 b3)
+__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
+    const auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = v[0];
+    b = v[1];
+}
+// (a0 a1 a2 a3), (b0 b1 b2 b3) -> (a0 b0 a2 b2), (a1 b1 a3 b3)
+__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
+    const auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = v[0];
+    b = v[1];
+}
+
+// Block u of the step for every lane: word g of its codes in x[u] and its scale
+// in d[u] (a 4 x 4 transpose over the lane rows, and a broadcast of each).
+__device__ __forceinline__ void st_spread(const StRaw& r, uint32_t (&x)[4], float (&d)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = r.w[i];
+    swap32(x[0], x[2]);
+    swap32(x[1], x[3]);
+    swap16(x[0], x[1]);
+    swap16(x[2], x[3]);
+    uint32_t a = __builtin_bit_cast(uint32_t, half_bits_to_float(r.d)), c = a;
+    swap32(a, c);                                      // (d0 d1 d0 d1), (d2 d3 d2 d3)
+    uint32_t b = a, e = c;
+    swap16(a, b);
+    swap16(c, e);
+    d[0] = __builtin_bit_cast(float, a);
+    d[1] = __builtin_bit_cast(float, b);
+    d[2] = __builtin_bit_cast(float, c);
+    d[3] = __builtin_bit_cast(float, e);
+}
+
+// q - 8 of word g of a block.  Q4_0: k = 4 g .. 4 g + 3 and 16 + 4 g .. (the
+// order the activations take in LDS); planes: k = 8 g .. 8 g + 7.
+template <int QT>
+__device__ __forceinline__ h8 st_codes(const Magic& mg, uint32_t x) {
+    if constexpr (QT == QT_PLANES) {
+        return bk_codes<QT_PLANES>(mg, BkRaw{x, 0, 0}, 0);
+    } else {
+        return bk_codes<QT_Q4_0>(mg, BkRaw{x, x >> 4, 0}, 0);
+    }
+}
+
+template <int QT, int MT, int NW>
+__global__ __launch_bounds__(64 * kBkWaves)
+void k_gemm_block_staged(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Waux,
+                         const uint16_t* __restrict__ A, int lda, void* __restrict__ C, int ldc, int out_f16, int M,
+                         int N, int K, int mcs) {
+    constexpr int KS = kBkWaves / NW;                  // parts of K, each with NW waves and stages of its own
+    constexpr int kStage = kStBlocks * MT * 1024;      // [block][row][lane row g] 16 bytes
+    constexpr int kPieces = kStBlocks * MT * 64;   // 16-byte pieces of a step
+    constexpr int PT = (kPieces + 64 * NW - 1) / (64 * NW);              // and per thread
+    __shared__ __attribute__((aligned(16))) uint8_t all[KS * 2 * kStage];
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * NW)), tid = (int)threadIdx.x - 64 * NW * kg;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t* const lds = all + kg * 2 * kStage;
+    // workgroup u runs on XCD u % 8: each XCD gets a contiguous run of units,
+    // the batch chunks of the same weight rows next to each other
+    const int n_units = (int)gridDim.x, xcd = (int)blockIdx.x & 7, q8 = n_units >> 3, rem8 = n_units & 7;
+    const int unit = xcd * q8 + min(xcd, rem8) + ((int)blockIdx.x >> 3);
+    const int nc = unit / mcs, m0 = 16 * MT * (unit - nc * mcs);
+    const int64_t nw = 16 * (NW * (int64_t)nc + wave) + r;         // this lane's weight row (output column)
+    // this group's steps; what they hold past the last block counts as zero
+    const int blocks = K >> 5, steps = (blocks + KS * kStBlocks - 1) / (KS * kStBlocks);
+    const int first = kg * steps * kStBlocks;
+    const int64_t n = min(nw, (int64_t)N - 1);
+    const uint8_t* const row = W + n * (QT == QT_Q4_0 ? 18 * (int64_t)blocks : 16 * (int64_t)blocks);
+    const uint8_t* const aux = QT == QT_Q4_0 ? nullptr : Waux + 2 * n * blocks;
+    // piece f of a step: row f / 16, block f / 4 % 4, eight k from 8 (f % 4)
+    const int pu = (tid >> 2) & 3, pp = tid & 3;
+    const uint16_t* src[PT];
+    uint32_t dst[PT];
+    bool own[PT];
+#pragma unroll
+    for (int i = 0; i < PT; i++) {
+        const int m = (tid >> 4) + 4 * NW * i;
+        own[i] = m < 16 * MT;
+        src[i] = A + (int64_t)min(m0 + m, M - 1) * lda + 8 * pp;
+        dst[i] = (uint32_t)(pu * MT * 1024 + m * 64 + (QT == QT_PLANES ? 16 * pp : 32 * (pp & 1) + 8 * (pp >> 1)));
+    }
+    const Magic mg = make_magic();
+    f4 acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) acc[i] = f4{0.f, 0.f, 0.f, 0.f};
+
+    // loads without a branch (it would drain them all): past the last block they
+    // read it again, and zeros are stored
+    auto load_a = [&](B16a2 (&a)[PT], int s) {
+        const int64_t k = 32 * (int64_t)min(first + kStBlocks * s + pu, blocks - 1);
+#pragma unroll
+        for (int i = 0; i < PT; i++) a[i] = *(const B16a2*)(src[i] + k);
+    };
+    auto store_a = [&](const B16a2 (&a)[PT], int s) {
+        uint8_t* const st = lds + (s & 1) * kStage;
+        const uint32_t on = first + kStBlocks * s + pu < blocks ? ~0u : 0u;
+#pragma unroll
+        for (int i = 0; i < PT; i++) {
+            if (!own[i]) continue;
+            if constexpr (QT == QT_PLANES) {
+                *(u4*)(st + dst[i]) = u4{a[i].x & on, a[i].y & on, a[i].z & on, a[i].w & on};
+            } else {
+                *(uint2*)(st + dst[i]) = uint2{a[i].x & on, a[i].y & on};
+                *(uint2*)(st + dst[i] + 16) = uint2{a[i].z & on, a[i].w & on};
+            }
+        }
+    };
+    // blocks past the last: its codes (finite) with a scale of zero
+    auto load_w = [&](StRaw& w, int s) {
+        w = st_load<QT>(row, aux, min(first + kStBlocks * s + g, blocks - 1));
+    };
+
+    B16a2 a[kStAhead][PT];
+    StRaw w[kStAhead];
+#pragma unroll
+    for (int j = 0; j < kStAhead; j++) {
+        load_w(w[j], j);
+        load_a(a[j], j);
+    }
+    store_a(a[0], 0);
+    load_a(a[0], kStAhead);
+    barrier_lds();
+    for (int s0 = 0; s0 < steps; s0 += kStAhead)
+#pragma unroll
+        for (int j = 0; j < kStAhead; j++) {
+            const int s = s0 + j;
+            if (s >= steps) break;
+            float d[kStBlocks];
+            uint32_t x[kStBlocks];
+            if (first + kStBlocks * s + g >= blocks) w[j].d = 0;   // (its codes are finite)
+            st_spread(w[j], x, d);
+            load_w(w[j], s + kStAhead);
+            store_a(a[(j + 1) % kStAhead], s + 1);
+            load_a(a[(j + 1) % kStAhead], s + 1 + kStAhead);
+            const uint8_t* const st = lds + (j & 1) * kStage + 64 * r + 16 * g;
+#pragma unroll
+            for (int u = 0; u < kStBlocks; u++) {
+                const h8 q = st_codes<QT>(mg, x[u]);
+                f4 p[MT];
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    p[i] = mfma16x16x32(*(const h8*)(st + (u * MT + i) * 1024), q, f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][e] = __builtin_fmaf(d[u], p[i][e], acc[i][e]);
+            }
+            barrier_lds();
+        }
+    if constexpr (KS == 2) {
+        // group 1's sums to group 0 (the last step's barrier freed the stages)
+        static_assert(KS * 2 * kStage >= NW * MT * 1024, "the hand-over fits the stages");
+        f4* const hand = (f4*)all + wave * MT * 64 + lane;
+        if (kg)
+#pragma unroll
+            for (int i = 0; i < MT; i++) hand[64 * i] = acc[i];
+        __syncthreads();
+        if (kg) return;
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[i] += hand[64 * i];
+    }
+    if (nw >= N) return;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int m = m0 + 16 * i + 4 * g + e;
+            if (m >= M) break;
+            const int64_t o = (int64_t)m * ldc + nw;
+            if (out_f16) ((_Float16*)C)[o] = (_Float16)acc[i][e];
+            else ((float*)C)[o] = acc[i][e];
+        }
+}
+
+struct BlockPlan { int MT, NT, NW, nb; int64_t grid; };   // NT = 0: the staged form, nb its batch chunks
 
 // Batch rows of a workgroup: all of them up to 64.  Two 16-row weight tiles
 // per workgroup (each activation load feeds two MFMAs) from 300 single ones on:
-// 313 (5000 rows, M = 1 / 8 / 20) 21.4 / 23.9 / 28.7 -> 20.4 / 21.5 / 24.6 us,
-// 1,565 (M = 300) 145 -> 120; 250 (2000 rows, M = 128) 18.6 -> 25.9.
+// 313 (5000 rows, M = 1 / 8 / 20) 21.4 / 23.9 / 28.7 -> 20.4 / 21.5 / 24.6 us;
+// 250 (2000 rows, M = 128) 18.6 -> 25.9.
+//
+// The staged form from 33 rows, where those tiles (64 batch rows x 32 weight
+// rows) take more than a workgroup per CU: 5000 x 5152 Q4_0 at M = 64 / 80 (157
+// / 314 tiles) 32.3 / 51 us direct, 35 / 32 staged; 4000 x 2976 at M = 128 / 129
+// (250 / 375) 19.7 / 32 and 22.5 / 20.  Short K from 1.5 per CU: 4500 x 672 at
+// M = 100 / 129 (282 / 423) 9.7 / 10.1 and 10.7 / 9.9.  Two groups of four waves
+// where their grid fits a round: 5000 x 5152 at M = 129 (237) 32 us, eight
+// waves 47; at M = 200 (316) 67 and 51.
 BlockPlan plan_block(const GemmArgs& g) {
     BlockPlan p;
     p.MT = std::min(4, (g.M + 15) / 16);
-    const int64_t mcs = (g.M + 16 * p.MT - 1) / (16 * p.MT), n16 = ((int64_t)g.N + 15) / 16;
+    const int64_t m16 = ((int64_t)g.M + 15) / 16, mcs = (m16 + p.MT - 1) / p.MT, n16 = ((int64_t)g.N + 15) / 16;
+    const int64_t cus = device_cus() > 0 ? device_cus() : 256, direct = mcs * ((n16 + 1) / 2);
+    if (g.M > 32 && direct > cus && (g.K >= 1024 || 2 * direct > 3 * cus)) {
+        p.MT = (int)((m16 + mcs - 1) / mcs);           // equal chunks
+        p.NT = 0;
+        p.NW = mcs * (((int64_t)g.N + 63) / 64) <= cus ? 4 : 8;
+        p.nb = (int)mcs;
+        p.grid = mcs * (((int64_t)g.N + 16 * p.NW - 1) / (16 * p.NW));
+        return p;
+    }
+    p.NW = kBkWaves;
     p.NT = mcs * n16 >= 300 ? 2 : 1;
     p.nb = (int)((n16 + p.NT - 1) / p.NT);
     p.grid = mcs * p.nb;
@@ -187,6 +424,12 @@ BlockPlan plan_block(const GemmArgs& g) {
 
 template <int QT, int MT>
 hipError_t launch_block(const GemmArgs& g, const BlockPlan& p, hipStream_t st) {
+    if constexpr (MT >= 3) if (p.NT == 0) {            // (33 rows are three tiles)
+        auto ks = p.NW == 8 ? k_gemm_block_staged<QT, MT, 8> : k_gemm_block_staged<QT, MT, 4>;
+        hipLaunchKernelGGL(ks, dim3((unsigned)p.grid), dim3(64 * kBkWaves), 0, st, g.W, g.Waux, g.A, g.lda, g.C, g.ldc,
+                           g.out_f16, g.M, g.N, g.K, p.nb);
+        return hipGetLastError();
+    }
     auto k = p.NT == 2 ? k_gemm_block<QT, MT, 2> : k_gemm_block<QT, MT, 1>;
     hipLaunchKernelGGL(k, dim3((unsigned)p.grid), dim3(64 * kBkWaves), 0, st, g.W, g.Waux, g.A, g.lda, g.C, g.ldc,
                        g.out_f16, g.M, g.N, g.K, p.nb);

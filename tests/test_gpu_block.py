@@ -68,3 +68,29 @@ def test_block_non_finite_rows(qt):
     assert (np.isfinite(C) == np.isfinite(D)).all()
     assert not np.isfinite(C[[2, 11, 19]]).any() and not np.isfinite(C[:, 3]).any()
     assert np.isfinite(np.delete(np.delete(C, [2, 11, 19], 0), 3, 1)).all()
+
+
+@pytest.mark.parametrize("qt", QTS, ids=lambda q: QT_NAME[q])
+@pytest.mark.parametrize("M,N,K,a_shift,w_shift,pad", [
+    (129, 2800, 1184, 1, 2, 1), (80, 4200, 1056, 0, 0, 0), (260, 2600, 416, 0, 0, 5), (300, 2600, 32, 0, 0, 0),
+    (300, 3301, 96, 0, 0, 3), (300, 3301, 1120, 3, 2, 1)])
+def test_block_staged_matches_simple(qt, M, N, K, a_shift, w_shift, pad):
+    """The form with the activations in LDS: three and four row tiles, K whole
+    and in two halves, block counts off its steps of four, one block."""
+    test_block_matches_simple(qt, M, N, K, a_shift, w_shift, pad)
+
+
+@pytest.mark.parametrize("qt", QTS, ids=lambda q: QT_NAME[q])
+@pytest.mark.parametrize("M,N,K", [(129, 2800, 1056), (300, 3301, 352)])
+def test_block_staged_non_finite_rows(qt, M, N, K):
+    """Infinite and NaN activations in a row's first and last block, which the
+    steps past the end read again, stay in their rows; an infinite last scale in
+    its column."""
+    w = O.gen_weights(qt, N, K, seed=9)
+    scales = w.W_aux if qt == O.Q4_0_PLANES else w.W.reshape(N, K // 32, 18)[:, :, :2].view(np.uint16)[..., 0]
+    scales[3, K // 32 - 1] = 0x7C00
+    A = O.gen_act(M, K, seed=10)
+    A[2, 7], A[11, 100], A[19, K - 1] = 0x7C00, 0x7E00, 0xFC00
+    C, D = run(qt, w, A, M, N, K), run(qt, w, A, M, N, K, algo=bf.ALGO_SIMPLE)
+    assert np.array_equal(np.isfinite(C), np.isfinite(D))
+    assert np.isfinite(np.delete(np.delete(C, [2, 11, 19], 0), 3, 1)).all()
