@@ -91,7 +91,7 @@ typedef enum {
     BF_ALGO_AUTO = 0,    /* pick by shape and M                                        */
     BF_ALGO_MFMA = 1,    /* v_mfma_f32_16x16x32_f16 over 16-row batch tiles            */
     BF_ALGO_DOT2 = 2,    /* v_dot2_f32_f16 lanes + cross-lane reduction (small M)      */
-    BF_ALGO_SIMPLE = 3,  /* one thread per output; any legal shape (slow, for odd K)   */
+    BF_ALGO_SIMPLE = 3,  /* one thread per output; any legal shape (slow)              */
     BF_ALGO_LDS = 4,     /* direct-to-LDS staged weights + MFMA (M <= 8; M <= 16 when A
                             fits in LDS; weight steps and A segments cycle through
                             rings when they do not fit)                               */
@@ -99,7 +99,7 @@ typedef enum {
     BF_ALGO_SPLIT = 6,   /* K split over workgroups, all operands resident in LDS (M <= 32);
                             uses a per-stream workspace allocated on first use          */
     BF_ALGO_DENSE = 7    /* all batch rows per workgroup, the weights streamed once
-                            (M <= 128 per launch; the default above 32 rows and on
+                            (M <= 128 per launch; the default at 33-128 rows and on
                             large matrices from 9 rows); one workgroup per CU over
                             equal shares of the row groups' K, split row groups
                             summed by a second launch through the same workspace      */
