@@ -7,6 +7,7 @@
 // evaluation agree and the only rounding is the final v_cvt_f16_f32 (RNE,
 // fp16 denormals preserved).
 #include "bf_formats.h"
+#include "bf_grid.h"
 #include "bf_launch.h"
 
 namespace bf {
@@ -44,7 +45,7 @@ __device__ __forceinline__ float elem_f32(int qt, const uint8_t* W, const uint8_
 }
 
 // One thread per 32-element group (a Q4_0 block or a Q4_K sub-block): weights
-// or output off their 16-byte boundaries.
+// or output off their 16-byte boundaries, and 2^35 weights or more.
 __global__ __launch_bounds__(256) void k_dequant_f16(int qt, const uint8_t* __restrict__ W,
                                                      const uint8_t* __restrict__ Waux,
                                                      uint16_t* __restrict__ out, int N, int K) {
@@ -116,10 +117,10 @@ __device__ __forceinline__ void dq_store(const Magic& mg, const DqUnit<QT>& u, u
 }
 
 template <int QT>
-__global__ __launch_bounds__(256) void k_dequant_f16_wide(const uint8_t* __restrict__ W,
-                                                          const uint8_t* __restrict__ Waux,
-                                                          uint16_t* __restrict__ out, int64_t units) {
-    const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
+__global__ __launch_bounds__(kDequantThreads) void k_dequant_f16_wide(const uint8_t* __restrict__ W,
+                                                                      const uint8_t* __restrict__ Waux,
+                                                                      uint16_t* __restrict__ out, int64_t units) {
+    const int64_t t = blockIdx.x * (int64_t)kDequantThreads + threadIdx.x;
     if (t >= units) return;
     DqUnit<QT> u;
     dq_load<QT>(u, W, Waux, t);
@@ -129,11 +130,11 @@ __global__ __launch_bounds__(256) void k_dequant_f16_wide(const uint8_t* __restr
 hipError_t dequant_f16(int qtype, const uint8_t* W, const uint8_t* Waux, uint16_t* out, int N, int K,
                        hipStream_t st) {
     const int64_t groups = (int64_t)N * (K >> 5), units = 4 * groups;
-    const int64_t wide = (units + 255) / 256;
-    if ((((uintptr_t)out | (qtype == QT_Q4_0 ? 0 : (uintptr_t)W)) & 15) == 0 && wide < (int64_t(1) << 31)) {
+    const int64_t wide = dequant_wide_grid(N, K);
+    if ((((uintptr_t)out | (qtype == QT_Q4_0 ? 0 : (uintptr_t)W)) & 15) == 0 && wide) {
         auto k = qtype == QT_Q4_K ? k_dequant_f16_wide<QT_Q4_K>
                  : qtype == QT_PLANES ? k_dequant_f16_wide<QT_PLANES> : k_dequant_f16_wide<QT_Q4_0>;
-        hipLaunchKernelGGL(k, dim3((unsigned)wide), dim3(256), 0, st, W, Waux, out, units);
+        hipLaunchKernelGGL(k, dim3((unsigned)wide), dim3(kDequantThreads), 0, st, W, Waux, out, units);
         return hipGetLastError();
     }
     int64_t blocks = (groups + 255) / 256;

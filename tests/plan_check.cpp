@@ -1,0 +1,44 @@
+// CPU check of the kernels' plans and grids (bus-fill_amd/csrc/bf_grid.h).
+// Every check prints what it expected on failure; exit status 0 when all hold.
+#include <cstdint>
+#include <cstdio>
+#include <cstring>
+
+#include "bf_grid.h"
+
+using namespace bf;
+
+namespace {
+
+int failures = 0;
+
+void expect(bool ok, const char* what, int64_t a = 0, int64_t b = 0, int64_t c = 0) {
+    if (ok) return;
+    failures++;
+    std::printf("FAIL %s (%lld, %lld, %lld)\n", what, (long long)a, (long long)b, (long long)c);
+}
+
+constexpr int64_t kItems = int64_t(1) << 32;           // work items of a launch along a dimension: fewer
+
+// The wide dequant grid covers every weight, is one HIP takes, and is given up
+// (for the general kernel) only where no such grid exists.
+void check_dequant() {
+    const int shapes[][2] = {{1, 32},        {17408, 5120},    {1 << 19, 1 << 15},  {1 << 20, 1 << 15},
+                             {1 << 25, 992}, {1 << 25, 1024},  {(1 << 25) - 1, 1024}, {(1 << 25) + 1, 1024},
+                             {1 << 30, 256}, {1 << 30, 8192},  {2147483647, 32}};
+    for (const auto& s : shapes) {
+        const int64_t weights = (int64_t)s[0] * s[1], need = (weights / 8 + 255) / 256, grid = dequant_wide_grid(s[0], s[1]);
+        if (need * 256 < kItems) expect(grid == need, "dequant grid covers the weights", s[0], s[1], grid);
+        else expect(grid == 0, "dequant grid above the launch limit", s[0], s[1], grid);
+    }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const char* only = argc > 1 ? argv[1] : "";
+    auto on = [&](const char* name) { return !*only || !std::strcmp(only, name); };
+    if (on("dequant")) check_dequant();
+    if (!failures) std::printf("ok\n");
+    return failures != 0;
+}
