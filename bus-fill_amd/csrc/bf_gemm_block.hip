@@ -25,9 +25,9 @@
 //
 // Where that takes more than a round of workgroups, k_gemm_block_staged passes
 // the activations through LDS (below).
-#include <algorithm>
 #include <type_traits>
 
+#include "bf_block_plan.h"
 #include "bf_formats.h"
 #include "bf_launch.h"
 #include "bf_lds.h"
@@ -35,7 +35,6 @@
 namespace bf {
 namespace {
 
-constexpr int kBkWaves = 8;
 constexpr int kBkUnroll = 4;             // blocks in flight per wave
 
 struct __attribute__((packed, aligned(2))) B8a2 { uint32_t x, y; };
@@ -388,38 +387,8 @@ void k_gemm_block_staged(const uint8_t* __restrict__ W, const uint8_t* __restric
         }
 }
 
-struct BlockPlan { int MT, NT, NW, nb; int64_t grid; };   // NT = 0: the staged form, nb its batch chunks
-
-// Batch rows of a workgroup: all of them up to 64.  Two 16-row weight tiles
-// per workgroup (each activation load feeds two MFMAs) from 300 single ones on:
-// 313 (5000 rows, M = 1 / 8 / 20) 21.4 / 23.9 / 28.7 -> 20.4 / 21.5 / 24.6 us;
-// 250 (2000 rows, M = 128) 18.6 -> 25.9.
-//
-// The staged form from 33 rows, where those tiles (64 batch rows x 32 weight
-// rows) take more than a workgroup per CU: 5000 x 5152 Q4_0 at M = 64 / 80 (157
-// / 314 tiles) 32.3 / 51 us direct, 35 / 32 staged; 4000 x 2976 at M = 128 / 129
-// (250 / 375) 19.7 / 32 and 22.5 / 20.  Short K from 1.5 per CU: 4500 x 672 at
-// M = 100 / 129 (282 / 423) 9.7 / 10.1 and 10.7 / 9.9.  Two groups of four waves
-// where their grid fits a round: 5000 x 5152 at M = 129 (237) 32 us, eight
-// waves 47; at M = 200 (316) 67 and 51.
-BlockPlan plan_block(const GemmArgs& g) {
-    BlockPlan p;
-    p.MT = std::min(4, (g.M + 15) / 16);
-    const int64_t m16 = ((int64_t)g.M + 15) / 16, mcs = (m16 + p.MT - 1) / p.MT, n16 = ((int64_t)g.N + 15) / 16;
-    const int64_t cus = device_cus() > 0 ? device_cus() : 256, direct = mcs * ((n16 + 1) / 2);
-    if (g.M > 32 && direct > cus && (g.K >= 1024 || 2 * direct > 3 * cus)) {
-        p.MT = (int)((m16 + mcs - 1) / mcs);           // equal chunks
-        p.NT = 0;
-        p.NW = mcs * (((int64_t)g.N + 63) / 64) <= cus ? 4 : 8;
-        p.nb = (int)mcs;
-        p.grid = mcs * (((int64_t)g.N + 16 * p.NW - 1) / (16 * p.NW));
-        return p;
-    }
-    p.NW = kBkWaves;
-    p.NT = mcs * n16 >= 300 ? 2 : 1;
-    p.nb = (int)((n16 + p.NT - 1) / p.NT);
-    p.grid = mcs * p.nb;
-    return p;
+BlockPlan plan_of(const GemmArgs& g) {
+    return plan_block(g.M, g.N, g.K, device_cus() > 0 ? device_cus() : 256);
 }
 
 template <int QT, int MT>
@@ -447,11 +416,12 @@ hipError_t dispatch_block(const GemmArgs& g, const BlockPlan& p, hipStream_t st)
 }  // namespace
 
 bool block_supports(const GemmArgs& g) {
-    return (g.qtype == QT_Q4_0 || g.qtype == QT_PLANES) && g.K % 32 == 0 && plan_block(g).grid < (int64_t(1) << 31);
+    return (g.qtype == QT_Q4_0 || g.qtype == QT_PLANES) && g.K % 32 == 0 &&
+           launch_fits(plan_of(g).grid, 64 * kBkWaves);
 }
 
 hipError_t gemm_block(const GemmArgs& g, hipStream_t st) {
-    const BlockPlan p = plan_block(g);
+    const BlockPlan p = plan_of(g);
     return g.qtype == QT_Q4_0 ? dispatch_block<QT_Q4_0>(g, p, st) : dispatch_block<QT_PLANES>(g, p, st);
 }
 

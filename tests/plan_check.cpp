@@ -1,9 +1,11 @@
-// CPU check of the kernels' plans and grids (bus-fill_amd/csrc/bf_grid.h).
+// CPU check of the kernels' plans and grids (bus-fill_amd/csrc/bf_grid.h,
+// bf_block_plan.h).
 // Every check prints what it expected on failure; exit status 0 when all hold.
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 
+#include "bf_block_plan.h"
 #include "bf_grid.h"
 
 using namespace bf;
@@ -33,12 +35,31 @@ void check_dequant() {
     }
 }
 
+// The block-wise kernel's workgroups cover the outputs, and a grid that HIP does
+// not take (64 kBkWaves threads per workgroup) is given up.
+void check_block_grid() {
+    const int shapes[][3] = {{1, 1, 32},          {37, 3001, 2336},     {300, 5000, 5152},   {129, 2800, 1184},
+                             {1, 1 << 28, 32},    {1, 1 << 27, 32},     {1, (1 << 28) - 32, 32}, {2147483647, 16, 32},
+                             {200000, 200000, 32}, {1 << 20, 1 << 13, 32}, {1 << 20, 1 << 16, 64}};
+    for (const auto& s : shapes) {
+        const int M = s[0], N = s[1];
+        const BlockPlan p = plan_block(M, N, s[2], 256);
+        const int64_t rows = 16 * (int64_t)(p.NT ? p.NT : p.NW), cols = ((int64_t)N + rows - 1) / rows;
+        expect(p.MT >= 1 && p.MT <= 4 && p.grid % cols == 0 && p.grid / cols * 16 * p.MT >= M, "block grid covers", M, N, p.grid);
+        const bool fits = launch_fits(p.grid, 64 * kBkWaves);
+        expect(fits == (p.grid * 64 * kBkWaves < kItems), "block grid against the launch limit", M, N, p.grid);
+    }
+    expect(!launch_fits(plan_block(1, 1 << 28, 32, 256).grid, 64 * kBkWaves), "2^28 weight rows: more than a launch");
+    expect(launch_fits(plan_block(1, (1 << 28) - 32, 32, 256).grid, 64 * kBkWaves), "2^28 - 32 weight rows: a launch");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const char* only = argc > 1 ? argv[1] : "";
     auto on = [&](const char* name) { return !*only || !std::strcmp(only, name); };
     if (on("dequant")) check_dequant();
+    if (on("block_grid")) check_block_grid();
     if (!failures) std::printf("ok\n");
     return failures != 0;
 }
