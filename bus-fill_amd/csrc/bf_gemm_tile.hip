@@ -34,16 +34,14 @@
 // * Measured (Q4_K, us per GEMM, before -> after): 17408 x 5120 at 512 / 2000
 //   rows 150-165 / 609-648 -> 108 / 355-369; 5120 x 17408 at 2000 rows
 //   572-606 -> 348-359; 5120 x 5120 at 300 / 512 rows 52-58 / 76-80 -> 35 / 43.
-#include <algorithm>
 #include <atomic>
 
 #include "bf_launch.h"
 #include "bf_lds.h"
+#include "bf_tile_plan.h"
 
 namespace bf {
 namespace {
-
-constexpr int kTlThreads = 512;          // eight waves, two per SIMD
 
 struct __attribute__((packed, aligned(2))) U2a2 { uint32_t x, y; };
 struct __attribute__((packed, aligned(2))) U4a2 { uint32_t x, y, z, w; };
@@ -491,52 +489,14 @@ __global__ __launch_bounds__(256) void k_tile_sum(const float* __restrict__ ws, 
     }
 }
 
-struct TilePlan {
-    int TA, NB, mt, F, R, S;
-    size_t part;                         // workspace bytes
-};
-
-// Microseconds of a plan, from measured launches (Q4_K): a super-group of each
-// tile shape takes `lo` up to 0.4 of the CUs busy and up to `hi` with all of
-// them (the chip is bound by power: fewer busy CUs clock higher), a round 6.5
-// for its start and end; the cut tiles' partials are written and read once,
-// and their sum is a launch of its own.
-double tile_cost(int TA, int NB, int nsg, int cus, int F, int R, int S, size_t piece) {
-    const double lo = NB == 2 ? 4.9 : TA == 4 ? 2.95 : TA == 3 ? 2.45 : 2.2;
-    const double hi = NB == 2 ? 7.6 : TA == 4 ? 4.1 : TA == 3 ? 3.3 : 2.4;
-    const int units = R * S, full = units / cus, rem = units % cus, n = (nsg + S - 1) / S;
-    const double last = lo + (hi - lo) * std::max(0.0, ((double)rem / cus - 0.4) / 0.6);
-    double c = F / cus * (nsg * hi + 6.5) + full * (n * hi + 6.5) + (rem ? n * last + 6.5 : 0.0);
-    if (S > 1) c += 3.0 + 2.0 * (double)units * (double)piece / 8e6;
-    return c;
-}
-
-bool plan_tile(const GemmArgs& g, TilePlan& p) {
-    if (g.M <= 128 || g.K % 256 || g.N < 1) return false;
+bool plan_of(const GemmArgs& g, TilePlan& p) {
     if ((int64_t)g.lda >= (1 << 22)) return false;     // activation offsets of a tile in 32 bits
-    const int cus = device_cus() > 0 ? device_cus() : 256, nsg = g.K / 256;
     // a caller's workspace of the size that 128-row launches of the dense kernel
     // take on this matrix serves here too
     GemmArgs slice = g;
     slice.M = 128;
     const size_t scratch = dense_supports(slice) ? dense_scratch_bytes(slice) : 0;
-    double best = 0;
-    for (int NB = 2; NB >= 1; NB--)
-        for (int TA = 4; TA >= (NB == 2 ? 4 : 2); TA--) {
-            const int64_t mt = (g.M + 64 * TA - 1) / (64 * TA), T = mt * ((g.N + 128 * NB - 1) / (128 * NB));
-            if (T >= (1 << 28)) continue;
-            const int F = (int)(T / cus * cus), R = (int)T - F;
-            const size_t piece = (size_t)64 * TA * 128 * NB * 4;
-            for (int S = 1; S <= std::min(nsg, 16); S++) {
-                if (S > 1 && (R == 0 || (size_t)R * S * piece > scratch)) break;
-                const double cost = tile_cost(TA, NB, nsg, cus, F, R, S, piece);
-                if (best == 0 || cost < best) {
-                    best = cost;
-                    p = TilePlan{TA, NB, (int)mt, F, R, S, S > 1 ? (size_t)R * S * piece : 0};
-                }
-            }
-        }
-    return best > 0;
+    return plan_tile(g.M, g.N, g.K, device_cus() > 0 ? device_cus() : 256, scratch, p);
 }
 
 template <int QT, int TA, int NB>
@@ -581,12 +541,12 @@ hipError_t dispatch_tile(const GemmArgs& g, const TilePlan& p, const Scratch* sc
 
 bool tile_supports(const GemmArgs& g) {
     TilePlan p;
-    return plan_tile(g, p);
+    return plan_of(g, p);
 }
 
 size_t tile_scratch_bytes(const GemmArgs& g) {
     TilePlan p;
-    return plan_tile(g, p) ? p.part : 0;
+    return plan_of(g, p) ? p.part : 0;
 }
 
 WsNeed tile_ws_need(const GemmArgs& g) {
@@ -597,7 +557,7 @@ WsNeed tile_ws_need(const GemmArgs& g) {
 
 hipError_t gemm_tile(const GemmArgs& g, const Scratch* scratch, hipStream_t st) {
     TilePlan p;
-    if (!plan_tile(g, p)) return hipErrorInvalidValue;
+    if (!plan_of(g, p)) return hipErrorInvalidValue;
     if (g.qtype == QT_PLANES) return dispatch_tile<QT_PLANES>(g, p, scratch, st);
     if (g.qtype == QT_Q4_0) return dispatch_tile<QT_Q4_0>(g, p, scratch, st);
     return dispatch_tile<QT_Q4_K>(g, p, scratch, st);

@@ -1,5 +1,5 @@
 // CPU check of the kernels' plans and grids (bus-fill_amd/csrc/bf_grid.h,
-// bf_block_plan.h).
+// bf_block_plan.h, bf_tile_plan.h).
 // Every check prints what it expected on failure; exit status 0 when all hold.
 #include <cstdint>
 #include <cstdio>
@@ -7,6 +7,7 @@
 
 #include "bf_block_plan.h"
 #include "bf_grid.h"
+#include "bf_tile_plan.h"
 
 using namespace bf;
 
@@ -53,6 +54,30 @@ void check_block_grid() {
     expect(launch_fits(plan_block(1, (1 << 28) - 32, 32, 256).grid, 64 * kBkWaves), "2^28 - 32 weight rows: a launch");
 }
 
+// Every tile plan covers the outputs, keeps its partials within the scratch on
+// offer and makes a grid that HIP takes; above that there is no plan.
+void check_tile_grid() {
+    const size_t offers[] = {0, size_t(1) << 20, size_t(32) << 20};
+    const int Ms[] = {129, 192, 257, 2000, 100000, 1 << 22, 1 << 24, 1 << 28, 2147483647}, Ns[] = {1, 128, 5120, 17408, 1 << 20, 1 << 28},
+              Ks[] = {256, 1280, 17408};
+    for (const size_t scratch : offers)
+        for (const int M : Ms)
+            for (const int N : Ns)
+                for (const int K : Ks) {
+                    TilePlan p{};
+                    if (!plan_tile(M, N, K, 256, scratch, p)) {
+                        const int64_t least = ((int64_t)M + 255) / 256 * (((int64_t)N + 255) / 256);
+                        expect((least + 16 * 256) * kTlThreads >= kItems, "no tile plan", M, N, K);
+                        continue;
+                    }
+                    const int64_t T = (int64_t)p.mt * (((int64_t)N + 128 * p.NB - 1) / (128 * p.NB));
+                    expect(p.F + (int64_t)p.R == T && (int64_t)p.mt * 64 * p.TA >= M, "tiles cover", M, N, K);
+                    expect(p.S >= 1 && p.S <= std::min(16, K / 256) && p.part <= scratch && (p.S == 1) == (p.part == 0),
+                           "tile cuts", M, N, K);
+                    expect((p.F + (int64_t)p.R * p.S) * kTlThreads < kItems, "tile grid against the launch limit", M, N, K);
+                }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -60,6 +85,7 @@ int main(int argc, char** argv) {
     auto on = [&](const char* name) { return !*only || !std::strcmp(only, name); };
     if (on("dequant")) check_dequant();
     if (on("block_grid")) check_block_grid();
+    if (on("tile_grid")) check_tile_grid();
     if (!failures) std::printf("ok\n");
     return failures != 0;
 }
