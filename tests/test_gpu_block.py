@@ -94,3 +94,27 @@ def test_block_staged_non_finite_rows(qt, M, N, K):
     C, D = run(qt, w, A, M, N, K), run(qt, w, A, M, N, K, algo=bf.ALGO_SIMPLE)
     assert np.array_equal(np.isfinite(C), np.isfinite(D))
     assert np.isfinite(np.delete(np.delete(C, [2, 11, 19], 0), 3, 1)).all()
+
+
+@pytest.mark.parametrize("qt", QTS, ids=lambda q: QT_NAME[q])
+@pytest.mark.parametrize("M,N,K", [(1, 40, 352), (20, 4900, 352), (129, 2800, 1056), (300, 3301, 352)])
+def test_block_infinite_scales(qt, M, N, K):
+    """Weights of infinite scale give what they give one by one: NaN where a code
+    is 8 or the signs differ, an infinity of the right sign where they agree."""
+    w = O.gen_weights(qt, N, K, seed=11)
+    blocks = K // 32
+    planes = qt == O.Q4_0_PLANES
+    scales = w.W_aux.reshape(N, blocks) if planes else w.W.reshape(N, blocks, 18)[:, :, :2].view(np.uint16)[..., 0]
+    codes = w.W.reshape(N, blocks, 16) if planes else w.W.reshape(N, blocks, 18)[:, :, 2:]
+    A = O.gen_act(M, K, seed=12)
+    A[0] &= 0x7FFF
+    A[0] |= 0x2000                                     # row 0: all positive, none zero
+    scales[3, blocks - 1], scales[5, 0], scales[7, 1], scales[9, blocks // 2] = 0x7C00, 0xFC00, 0x7E00, 0x7C00
+    codes[5, 0] = 0x99                                 # q - 8 = 1 throughout: -inf times a positive row
+    codes[9, blocks // 2] = 0x77                       # -1 throughout
+    for otype in (bf.OUT_F32, bf.OUT_F16):
+        C, D = (run(qt, w, A, M, N, K, algo=a, otype=otype) for a in (bf.ALGO_AUTO, bf.ALGO_SIMPLE))
+        odd = ~np.isfinite(D)
+        assert (odd == ~np.isfinite(C)).all() and odd[:, [3, 5, 7, 9]].all() and odd.sum() == 4 * M
+        assert np.array_equal(C[odd], D[odd], equal_nan=True)
+        assert C[0, 5] == -np.inf and C[0, 9] == -np.inf and np.isnan(C[0, [3, 7]]).all()
