@@ -48,4 +48,10 @@ inline BlockPlan plan_block(int M, int N, int K, int cus) {
     return p;
 }
 
+// One block per weight row and one batch row: from some 2^18 weight rows on, a
+// thread per output is faster (Q4_0 / planes, a thread per output against here,
+// us: 131072 rows 7.5 / 9.4 and 7.2 / 7.0, 262144 rows 11.8 / 12.9 and 14.6 /
+// 14.4, 1000000 rows 39 / 40 and 52 / 49; at two batch rows 73 / 76 and 56 / 53).
+inline bool block_slower(int M, int N, int K) { return M == 1 && K == 32 && N >= 200000; }
+
 }  // namespace bf

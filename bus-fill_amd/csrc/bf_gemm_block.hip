@@ -462,7 +462,7 @@ hipError_t dispatch_block(const GemmArgs& g, const BlockPlan& p, hipStream_t st)
 }  // namespace
 
 bool block_supports(const GemmArgs& g) {
-    return (g.qtype == QT_Q4_0 || g.qtype == QT_PLANES) && g.K % 32 == 0 &&
+    return (g.qtype == QT_Q4_0 || g.qtype == QT_PLANES) && g.K % 32 == 0 && !block_slower(g.M, g.N, g.K) &&
            launch_fits(plan_of(g).grid, 64 * kBkWaves);
 }
 

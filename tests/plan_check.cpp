@@ -78,6 +78,15 @@ void check_tile_grid() {
                 }
 }
 
+// The block-wise kernel only where it is the faster one.
+void check_block_choice() {
+    expect(block_slower(1, 262144, 32) && block_slower(1, 1000000, 32), "one row, one block, many weight rows: a thread per output");
+    for (const int M : {1, 2, 16, 300})
+        for (const int N : {16, 5000, 131072})
+            for (const int K : {32, 64, 2336}) expect(!block_slower(M, N, K), "block-wise", M, N, K);
+    expect(!block_slower(2, 1000000, 32) && !block_slower(1, 1000000, 64), "two rows or two blocks: block-wise");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -85,6 +94,7 @@ int main(int argc, char** argv) {
     auto on = [&](const char* name) { return !*only || !std::strcmp(only, name); };
     if (on("dequant")) check_dequant();
     if (on("block_grid")) check_block_grid();
+    if (on("block_choice")) check_block_choice();
     if (on("tile_grid")) check_tile_grid();
     if (!failures) std::printf("ok\n");
     return failures != 0;
