@@ -86,14 +86,13 @@ namespace {
 // wait for the release flag, then load A with device-scope loads.  dep_users
 // workgroups wait; the last of them past its wait clears the words.  CO: C is
 // stored with device-scope stores (written through to the point of coherence:
-// the output is such a dependency's A).  AF (with BD or AC): A is fp32 rows
-// (lda in floats), rounded to fp16 as the compute waves load them.  EA (plans
-// whose steps all have a slot of their own, no step ring): each loader issues
-// the first group's step before the rest of its setup.
-constexpr int kAfBatch = 2;              // activation instructions of a wave in flight (AF)
-
+// the output is such a dependency's A).  AF > 0 (with BD or AC): A is fp32
+// rows (lda in floats), rounded to fp16 as the compute waves load them, AF of a
+// wave's load instructions in flight together.  EA (plans whose steps all have a
+// slot of their own, no step ring): each loader issues the first group's step
+// before the rest of its setup.
 template <int QT, int G, int MT, int NC, int NL, bool BD, bool RG, bool AC, bool SW = false, bool DEP = false,
-          bool CO = false, bool AF = false, bool EA = false>
+          bool CO = false, int AF = 0, bool EA = false>
 __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* __restrict__ W,
                                          const uint16_t* __restrict__ A, int lda, int M, int N, int K, int nsub,
                                          int nslot, int na, int win, const uint8_t* __restrict__ Waux,
@@ -421,7 +420,7 @@ __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* _
             } else if constexpr (SW) {
                 if (P < nsg * 33)
                     *(u4*)(lds + kFlagBytes + 1024 * i + 16 * lane) = swiglu8(A + 256 * sg + 8 * c, A + K + 256 * sg + 8 * c);
-            } else if constexpr (AF) {
+            } else if constexpr (AF > 0) {
                 if (P < nsg * 33)
                     *(u4*)(lds + kFlagBytes + 1024 * i + 16 * lane) =
                         f32x8_to_f16((const float*)(const void*)A + 256 * sg + 8 * c);
@@ -450,16 +449,13 @@ __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* _
             on = P < (uint32_t)PA && c < 32;
             return (int64_t)min((int)m, M - 1) * lda + 256 * (G * sg + gg) + 8 * min((int)c, 31);
         };
-        if constexpr (AF) {
-            // fp32 rows through registers: kAfBatch instructions' loads in flight
-            // together (5120^2 Q4_K at batch 2 / 8: 7.1 / 10.1 us with two, 7.6 /
-            // 10.1 with four, 8.7 / 10.1 with eight)
-            for (int f0 = cw; f0 < nsteps * IA; f0 += kAfBatch * NC) {
-                f4 v[kAfBatch][2];
-                int sg[kAfBatch], i[kAfBatch];
-                bool on[kAfBatch];
+        if constexpr (AF > 1) {
+            for (int f0 = cw; f0 < nsteps * IA; f0 += AF * NC) {
+                f4 v[AF][2];
+                int sg[AF], i[AF];
+                bool on[AF];
 #pragma unroll
-                for (int u = 0; u < kAfBatch; u++) {
+                for (int u = 0; u < AF; u++) {
                     const float* src = (const float*)(const void*)A + piece(f0 + u * NC, sg[u], i[u], on[u]);
                     on[u] = on[u] && f0 + u * NC < nsteps * IA;
                     if (on[u]) {
@@ -468,13 +464,13 @@ __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* _
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < kAfBatch; u++)
+                for (int u = 0; u < AF; u++)
                     if (on[u])
                         *(u4*)(lds + kFlagBytes + sg[u] * seg_bytes + (i[u] << 10) + 16 * lane) =
                             f32x8_to_f16(v[u][0], v[u][1]);
             }
         }
-        for (int f = cw; !AF && f < nsteps * IA; f += NC) {
+        for (int f = cw; AF <= 1 && f < nsteps * IA; f += NC) {
             int sg, i;
             bool on;
             const int64_t elem = piece(f, sg, i, on);
@@ -483,6 +479,10 @@ __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* _
                 if (on) *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) = swiglu_dep(elem);
             } else if constexpr (SW) {
                 if (on) *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) = swiglu8(src, src + K);
+            } else if constexpr (AF == 1) {
+                if (on)
+                    *(u4*)(lds + kFlagBytes + sg * seg_bytes + (i << 10) + 16 * lane) =
+                        f32x8_to_f16((const float*)(const void*)A + elem);
             } else {
                 if (on) dma16(src, lds0 + (uint32_t)(kFlagBytes + sg * seg_bytes + (i << 10)));
             }
@@ -864,7 +864,7 @@ __device__ __forceinline__ void lds_body(int bid, uint8_t* lds, const uint8_t* _
 // started, so the loaders' second group of steps and every step marker would
 // wait for it.  mo = M | out_f16 << 8 | nsub << 16 | win << 24, sl = nslot |
 // na << 16 (lds_packed_args).
-template <int QT, int G, int MT, int NC, int NL, bool BD, bool RG, bool AC = false, bool SW = false, bool AF = false,
+template <int QT, int G, int MT, int NC, int NL, bool BD, bool RG, bool AC = false, bool SW = false, int AF = 0,
           bool EA = false>
 __global__ __launch_bounds__(64 * (NC + NL))
 void k_gemm_lds(const uint8_t* __restrict__ W, const uint16_t* __restrict__ A, const uint8_t* __restrict__ Waux,
@@ -920,7 +920,7 @@ bool lds_packed_args(const GemmArgs& g, const LdsPlan& p, uint32_t& mo, uint32_t
     return true;
 }
 
-template <int QT, int G, int MT, bool BD = false, bool RG = false, bool AC = false, bool SW = false, bool AF = false,
+template <int QT, int G, int MT, bool BD = false, bool RG = false, bool AC = false, bool SW = false, int AF = 0,
           bool EA = false>
 hipError_t launch_lds(const GemmArgs& g, const LdsPlan& p, hipStream_t st) {
     auto k = k_gemm_lds<QT, G, MT, kNC, kNL, BD, RG, AC, SW, AF, EA>;
@@ -949,14 +949,20 @@ hipError_t dispatch_lds(const GemmArgs& g, const LdsPlan& p, hipStream_t st) {
     // 8.16 us)
     const bool ea = QT == QT_Q4_K && p.nslot >= p.nsub * (g.K / (256 * p.G));
     if (g.a_f32) {
-        if (p.BD) return ea ? launch_lds<QT, 4, 1, true, false, false, false, true, true>(g, p, st)
-                            : launch_lds<QT, 4, 1, true, false, false, false, true>(g, p, st);
-        if (p.MT == 2) return ea ? launch_lds<QT, 4, 2, false, false, true, false, true, true>(g, p, st)
-                                 : launch_lds<QT, 4, 2, false, false, true, false, true>(g, p, st);
-        return ea ? launch_lds<QT, 4, 1, false, false, true, false, true, true>(g, p, st)
-                  : launch_lds<QT, 4, 1, false, false, true, false, true>(g, p, st);
+        // A wave's load instructions in flight: one where the plan's fp16 form has
+        // the compute waves load A too (small A, up to three instructions a wave:
+        // the second one's address delays the first), two above (5120^2 Q4_K at
+        // batch 8: 10.1 us with two, four or eight).
+        if (p.BD) return ea ? launch_lds<QT, 4, 1, true, false, false, false, 1, true>(g, p, st)
+                            : launch_lds<QT, 4, 1, true, false, false, false, 1>(g, p, st);
+        if (p.MT == 2) return ea ? launch_lds<QT, 4, 2, false, false, true, false, 2, true>(g, p, st)
+                                 : launch_lds<QT, 4, 2, false, false, true, false, 2>(g, p, st);
+        if (p.AC) return ea ? launch_lds<QT, 4, 1, false, false, true, false, 1, true>(g, p, st)
+                            : launch_lds<QT, 4, 1, false, false, true, false, 1>(g, p, st);
+        return ea ? launch_lds<QT, 4, 1, false, false, true, false, 2, true>(g, p, st)
+                  : launch_lds<QT, 4, 1, false, false, true, false, 2>(g, p, st);
     }
-    if (p.BD) return ea ? launch_lds<QT, 4, 1, true, false, false, false, false, true>(g, p, st)
+    if (p.BD) return ea ? launch_lds<QT, 4, 1, true, false, false, false, 0, true>(g, p, st)
                         : launch_lds<QT, 4, 1, true>(g, p, st);
     if (p.RG) {
         if (p.G == 4 && p.MT == 1) return launch_lds<QT, 4, 1, false, true>(g, p, st);
@@ -964,11 +970,11 @@ hipError_t dispatch_lds(const GemmArgs& g, const LdsPlan& p, hipStream_t st) {
         if (p.G == 2 && p.MT == 1) return launch_lds<QT, 2, 1, false, true>(g, p, st);
         return hipErrorInvalidValue;                    // no ring kernel of this shape
     }
-    if (p.AC) return ea ? launch_lds<QT, 4, 1, false, false, true, false, false, true>(g, p, st)
+    if (p.AC) return ea ? launch_lds<QT, 4, 1, false, false, true, false, 0, true>(g, p, st)
                         : launch_lds<QT, 4, 1, false, false, true>(g, p, st);
-    if (p.G == 4 && p.MT == 1) return ea ? launch_lds<QT, 4, 1, false, false, false, false, false, true>(g, p, st)
+    if (p.G == 4 && p.MT == 1) return ea ? launch_lds<QT, 4, 1, false, false, false, false, 0, true>(g, p, st)
                                          : launch_lds<QT, 4, 1>(g, p, st);
-    if (p.G == 4 && p.MT == 2) return ea ? launch_lds<QT, 4, 2, false, false, false, false, false, true>(g, p, st)
+    if (p.G == 4 && p.MT == 2) return ea ? launch_lds<QT, 4, 2, false, false, false, false, 0, true>(g, p, st)
                                          : launch_lds<QT, 4, 2>(g, p, st);
     if (p.G == 2 && p.MT == 1) return launch_lds<QT, 2, 1>(g, p, st);
     return launch_lds<QT, 1, 1>(g, p, st);
@@ -1206,14 +1212,14 @@ bool lds_supports(const GemmArgs& g) {
     return choose_lds(lds_shape(g), p);
 }
 
-// fp32 rows (the ggml hook): plans that keep all of A in LDS, in the form whose
-// compute waves load it.  Up to batch 8 that costs no more than the staging launch
-// the rows would otherwise take, although the loaders' way is faster for fp16
-// rows (Q4_K, us, batch 3 / 5 / 8: 5120^2 10.4 / 11.0 / 11.3 -> 7.6 / 8.8 /
-// 10.1; 17408 x 5120 16.6 / 18.5 / 19.1 -> 13.3 / 15.9 / 17.8; 3000 x 8192
-// 10.3 / 11.6 / 13.2 -> 7.8 / 9.8 / 13.3).
+// fp32 rows (the ggml hook): up to batch 8 the compute waves' loads cost less
+// than the staging launch the rows would otherwise take, although the loaders'
+// way is faster for fp16 rows (Q4_K, us, staged -> here, batch 3 / 5 / 8: 5120 x
+// 5120 9.1 / 10.1 / 10.4 -> 7.1 / 8.3 / 9.4; 17408 x 5120 16.8 / 19.0 / 19.4 ->
+// 13.5 / 16.0 / 17.5; batch 3 / 5 / 6 at 3000 x 8192, whose batches 7 and 8 keep
+// no plan with all of A: 9.6 / 10.8 / 11.0 -> 7.3 / 9.3 / 9.6).
 bool lds_f32_plan(const GemmArgs& g, LdsPlan& p) {
-    return choose_lds(lds_shape(g), p) && (p.BD || (!p.RG && p.G == 4));
+    return choose_lds(lds_shape(g), p) && lds_f32_form(p);
 }
 
 bool lds_f32_supports(const GemmArgs& g) {

@@ -170,4 +170,8 @@ inline bool choose_lds(const LdsShape& g, LdsPlan& p) {
     return false;
 }
 
+// The ggml hook's fp32 rows: plans that keep all of A in LDS run in the form
+// whose compute waves load it (as AC), rounding it on the way.
+inline bool lds_f32_form(const LdsPlan& p) { return p.BD || (!p.RG && p.G == 4); }
+
 }  // namespace bf

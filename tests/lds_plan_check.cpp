@@ -19,6 +19,8 @@
 //     the sub-tile's last step, after its own steps).
 //   AC plans (small A): the compute waves load all of A before the barrier and
 //     wait for it (no dependence on the loaders), the loaders stream weights only.
+//     fp32 rows run every plan that keeps all of A in this form (two m-tiles and
+//     step rings among them), so those plans are checked in it too.
 // Bounded waits: every wait of the kernel gives up after a bound, marks the
 // workgroup poisoned (an LDS word every store of a result reads first) and
 // goes on.  Runs with a planted missing producer (a step marker, one loader's
@@ -517,7 +519,7 @@ int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "--self-test") == 0) return self_test();
     const int Ns[] = {1, 77, 512, 600, 1024, 3072, 4096, 5120, 7168, 13824, 17408, 27648};
     const int Ks[] = {256, 1024, 2048, 3072, 4096, 5120, 8192, 13824, 17408, 24576, 27648};
-    int plans = 0, rings = 0, aring = 0, ac = 0, runs = 0, drop_plans = 0;
+    int plans = 0, rings = 0, aring = 0, ac = 0, runs = 0, drop_plans = 0, f32 = 0, f32_rings = 0;
     for (int q = 0; q < 2; q++)
         for (int M = 1; M <= 16; M++)
             for (int N : Ns)
@@ -547,11 +549,27 @@ int main(int argc, char** argv) {
                             run_drops(g, p, nsteps, (uint64_t)(M * 131 + N) * 17u + K);
                             drop_plans++;
                         }
+                        // fp32 rows: the same plan with A loaded by the compute waves
+                        if (M <= 8 && lds_f32_form(p) && !p.BD && !p.AC) {
+                            LdsPlan f = p;
+                            f.AC = true;
+                            for (int mode = 0; mode < 3; mode++) {
+                                Model m(g, f, nsteps);
+                                m.run((uint64_t)mode * 7919u + (uint64_t)(M * 131 + N) * 17u + K, mode);
+                            }
+                            if (ring || f32 % 5 == 0) run_drops(g, f, nsteps, (uint64_t)(M * 131 + N) * 19u + K);
+                            f32++;
+                            f32_rings += ring && p.MT == 2;
+                        }
                     } catch (const std::exception& e) {
                         std::printf("FAIL %s\n", e.what());
                         return 1;
                     }
                 }
+    if (f32 < 400 || f32_rings < 20) {
+        std::printf("FAIL fp32-row plans: %d, %d of them two m-tiles with a step ring\n", f32, f32_rings);
+        return 1;
+    }
     std::printf("ok: %d plans (%d with a step ring, %d with windows / activation ring), %d model runs, %d AC, "
                 "%d with missing producers\n", plans, rings, aring, runs, ac, drop_plans);
     return 0;

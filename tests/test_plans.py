@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+import busfill as bf
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -25,3 +27,20 @@ def checker(tmp_path_factory):
 def test_plans(checker, part):
     r = subprocess.run([checker, part], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_fp32_rows_inside_the_gemm():
+    """ggml hook: up to eight fp32 rows go to the LDS kernel itself (no
+    workspace) wherever its plan keeps all of A; nine rows, and plans with an
+    activation ring, are staged."""
+    fmts = {"q4_0": (bf.GGML_Q4_0, 32, 18), "q4_k": (bf.GGML_Q4_K, 256, 144)}
+    most = {(3000, 8192, "q4_0"): 7, (300, 8192, "q4_k"): 7, (3000, 8192, "q4_k"): 6}
+    for fmt, (gt, blk, bb) in fmts.items():
+        for N, K in ((1, 1024), (77, 2048), (5120, 5120), (17408, 1024), (17408, 5120), (27648, 5120), (300, 8192),
+                     (3000, 8192)):
+            for M in range(1, 10):
+                views = (bf.ggml_tensor(gt, 1 << 20, (K, N), (bb, K // blk * bb)),
+                         bf.ggml_tensor(bf.GGML_F32, 1 << 24, (K, M), (4, 4 * K)),
+                         bf.ggml_tensor(bf.GGML_F32, 1 << 28, (N, M), (4, 4 * N)))
+                inside = bf.ggml_mul_mat_workspace_bytes(*views) == 0
+                assert inside == (M <= most.get((N, K, fmt), 8)), (fmt, N, K, M)
