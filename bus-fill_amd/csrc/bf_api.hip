@@ -191,9 +191,10 @@ bf_status plan_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uint
         return g;
     };
     // Above 128 rows the tile kernel (17408 x 5120 at 512 rows: 150-165 us in
-    // dense launches of 128 rows, 108 here); up to there the dense kernel is
-    // faster (at 128 rows 38.0 us against 39.2 on 5120 x 17408, 38.7 against
-    // 42.5 on 17408 x 5120, both with tiles of 128 rows and K cut to fill the chip).
+    // dense launches of 128 rows, 108 here), but on some matrices up to 256 rows
+    // (slices_faster); up to 128 the dense kernel is faster (at 128 rows 38.0 us
+    // against 39.2 on 5120 x 17408, 38.7 against 42.5 on 17408 x 5120, both with
+    // tiles of 128 rows and K cut to fill the chip).
     if (algo == BF_ALGO_AUTO && M > kMaxMPerLaunch) {
         const bf::GemmArgs g = args(0, M);
         if (fast_eligible(g) && bf::tile_supports(g)) {

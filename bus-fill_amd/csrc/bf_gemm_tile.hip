@@ -541,7 +541,12 @@ hipError_t dispatch_tile(const GemmArgs& g, const TilePlan& p, const Scratch* sc
 
 bool tile_supports(const GemmArgs& g) {
     TilePlan p;
-    return plan_of(g, p);
+    if (!plan_of(g, p)) return false;
+    GemmArgs slice = g;
+    slice.M = 128;
+    return !(dense_supports(slice) &&
+             slices_faster(g.M, g.N, g.K, device_cus() > 0 ? device_cus() : 256,
+                           g.qtype == QT_PLANES ? 1.12 : g.qtype == QT_Q4_0 ? 1.08 : 1.04, p));
 }
 
 size_t tile_scratch_bytes(const GemmArgs& g) {

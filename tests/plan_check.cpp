@@ -87,6 +87,30 @@ void check_block_choice() {
     expect(!block_slower(2, 1000000, 32) && !block_slower(1, 1000000, 64), "two rows or two blocks: block-wise");
 }
 
+// Tiles or 128-row launches, at measured points on both sides of the rule (256
+// CUs, 32 MB of scratch; formats by their factor).
+void check_tile_choice() {
+    const double q4k = 1.04, q40 = 1.08, planes = 1.12;
+    struct Point { int M, N, K; double slow; bool slices; };
+    const Point points[] = {
+        {129, 17408, 5120, q4k, true},    {136, 17408, 5120, q4k, true},    {192, 17408, 5120, q4k, false},
+        {160, 17408, 5120, q40, true},    {192, 17408, 5120, q40, false},   {193, 17408, 5120, planes, true},
+        {256, 17408, 5120, q4k, false},   {257, 17408, 5120, planes, false}, {160, 17408, 17408, q4k, true},
+        {193, 17408, 17408, q4k, true},   {256, 17408, 17408, q40, false},  {129, 28672, 4096, planes, false},
+        {129, 32000, 4096, q4k, false},   {144, 16384, 4096, q40, false},   {160, 16896, 2816, planes, false},
+        {129, 5120, 5120, q4k, true},     {140, 5120, 5120, q4k, false},    {132, 2048, 8192, planes, true},
+        {136, 2048, 8192, q4k, false},    {136, 6144, 4096, q40, true},     {144, 4096, 4096, q4k, false},
+        {129, 1024, 1024, q4k, false},    {129, 256, 17408, planes, false}, {129, 5120, 17408, q4k, false},
+        {129, 4042, 3328, q40, false},    {512, 17408, 5120, planes, false}, {256, 2048, 8192, q4k, false},
+        {300, 5120, 5120, q4k, false},    {129, 8870, 4864, q4k, false},    {130, 11921, 1792, planes, false},
+        {2000, 17408, 17408, q4k, false}};
+    for (const Point& x : points) {
+        TilePlan p{};
+        expect(plan_tile(x.M, x.N, x.K, 256, size_t(32) << 20, p), "a tile plan", x.M, x.N, x.K);
+        expect(slices_faster(x.M, x.N, x.K, 256, x.slow, p) == x.slices, x.slices ? "128-row launches" : "tiles", x.M, x.N, x.K);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -96,6 +120,7 @@ int main(int argc, char** argv) {
     if (on("block_grid")) check_block_grid();
     if (on("block_choice")) check_block_choice();
     if (on("tile_grid")) check_tile_grid();
+    if (on("tile_choice")) check_tile_choice();
     if (!failures) std::printf("ok\n");
     return failures != 0;
 }

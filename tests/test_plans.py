@@ -23,7 +23,7 @@ def checker(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("part", ["dequant", "block_grid", "block_choice", "tile_grid"])
+@pytest.mark.parametrize("part", ["dequant", "block_grid", "block_choice", "tile_grid", "tile_choice"])
 def test_plans(checker, part):
     r = subprocess.run([checker, part], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
