@@ -1,8 +1,12 @@
 // CPU check of the kernels' plans and grids (bus-fill_amd/csrc/bf_grid.h,
 // bf_block_plan.h, bf_tile_plan.h).
 // Every check prints what it expected on failure; exit status 0 when all hold.
+// `plan_check tile M N K` and `plan_check block M N K` print a plan on 256 CUs
+// (TA NB F R S, with the scratch of a 128-row dense launch, and whether a format
+// of factor 1 would take 128-row launches instead; MT NT NW).
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 
 #include "bf_block_plan.h"
@@ -114,6 +118,19 @@ void check_tile_choice() {
 }  // namespace
 
 int main(int argc, char** argv) {
+    if (argc == 5) {
+        const int M = std::atoi(argv[2]), N = std::atoi(argv[3]), K = std::atoi(argv[4]);
+        if (!std::strcmp(argv[1], "block")) {
+            const BlockPlan b = plan_block(M, N, K, 256);
+            std::printf("%d %d %d\n", b.MT, b.NT, b.NW);
+            return 0;
+        }
+        TilePlan p{};
+        const int64_t units = ((int64_t)N + 127) / 128 * (K / 256);
+        if (!plan_tile(M, N, K, 256, (size_t)std::min<int64_t>(units, 256) * 2 * 128 * 128 * 4, p)) return 1;
+        std::printf("%d %d %d %d %d %d\n", p.TA, p.NB, p.F, p.R, p.S, (int)slices_faster(M, N, K, 256, 1.0, p));
+        return 0;
+    }
     const char* only = argc > 1 ? argv[1] : "";
     auto on = [&](const char* name) { return !*only || !std::strcmp(only, name); };
     if (on("dequant")) check_dequant();

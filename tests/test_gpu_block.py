@@ -18,6 +18,17 @@ QTS = [O.Q4_0_PLANES, O.Q4_0]
 QT_NAME = {O.Q4_0_PLANES: "planes", O.Q4_0: "q4_0"}
 
 
+# (M, N, K): (MT, NT, NW), the form of the kernel it runs (16 MT batch rows x 16 NT weight rows; NT = 0: activations
+# through LDS, NW of the eight waves over weight rows); tests/test_plans.py holds the plans to it on the CPU.
+FORMS = {
+    (1, 1, 32): (1, 1, 8), (16, 15, 96): (1, 1, 8), (17, 33, 288): (2, 1, 8), (48, 300, 160): (3, 1, 8),
+    (64, 17, 1184): (4, 1, 8), (65, 100, 2336): (4, 1, 8), (1, 4900, 416): (1, 2, 8), (129, 1700, 96): (4, 2, 8),
+    (5, 70, 512): (1, 1, 8), (140, 64, 1024): (4, 1, 8), (20, 5000, 416): (2, 2, 8), (40, 4900, 416): (3, 2, 8),
+    (129, 2800, 1184): (3, 0, 4), (80, 4200, 1056): (3, 0, 4), (260, 2600, 416): (4, 0, 4), (300, 2600, 32): (4, 0, 4),
+    (300, 3301, 96): (4, 0, 8), (300, 3301, 1120): (4, 0, 8), (129, 6000, 1120): (3, 0, 8),
+}
+
+
 def to_dev(a, shift=0):
     """On the device, `shift` elements into a buffer of its own."""
     t = torch.from_numpy(np.ascontiguousarray(a).view(np.int16 if a.dtype == np.uint16 else a.dtype))
@@ -41,7 +52,7 @@ def run(qt, w, A, M, N, K, *, algo=bf.ALGO_AUTO, a_shift=0, w_shift=0, pad=0, ot
 @pytest.mark.parametrize("M,N,K,a_shift,w_shift,pad", [
     (1, 1, 32, 0, 0, 0), (16, 15, 96, 0, 0, 0), (17, 33, 288, 0, 0, 3), (48, 300, 160, 1, 0, 0), (64, 17, 1184, 0, 0, 5),
     (65, 100, 2336, 3, 2, 1), (1, 4900, 416, 0, 0, 0), (129, 1700, 96, 0, 0, 0), (5, 70, 512, 1, 0, 1),
-    (140, 64, 1024, 0, 2, 0)])
+    (140, 64, 1024, 0, 2, 0), (20, 5000, 416, 0, 0, 0), (40, 4900, 416, 0, 0, 1)])
 def test_block_matches_simple(qt, M, N, K, a_shift, w_shift, pad):
     w = O.gen_weights(qt, N, K, seed=N + K)
     A = O.gen_act(M, K, seed=M + K)
@@ -73,7 +84,7 @@ def test_block_non_finite_rows(qt):
 @pytest.mark.parametrize("qt", QTS, ids=lambda q: QT_NAME[q])
 @pytest.mark.parametrize("M,N,K,a_shift,w_shift,pad", [
     (129, 2800, 1184, 1, 2, 1), (80, 4200, 1056, 0, 0, 0), (260, 2600, 416, 0, 0, 5), (300, 2600, 32, 0, 0, 0),
-    (300, 3301, 96, 0, 0, 3), (300, 3301, 1120, 3, 2, 1)])
+    (300, 3301, 96, 0, 0, 3), (300, 3301, 1120, 3, 2, 1), (129, 6000, 1120, 0, 0, 0)])
 def test_block_staged_matches_simple(qt, M, N, K, a_shift, w_shift, pad):
     """The form with the activations in LDS: three and four row tiles, K whole
     and in two halves, block counts off its steps of four, one block."""

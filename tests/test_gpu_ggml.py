@@ -90,7 +90,7 @@ CASES = [
     (QK, F32, 96, 33, 256, 3, 1, 1, 1, "contig"),
     (Q0, F32, 96, 16, 512, 2, 2, 2, 1, "permuted"),
     (QK, F16, 64, 9, 256, 4, 3, 2, 3, "permuted"),      # fp16 rows ne2 rows apart: in place
-    (QK, F32, 128, 130, 256, 1, 1, 1, 1, "contig"),     # above 128 rows (sliced)
+    (QK, F32, 128, 130, 256, 1, 1, 1, 1, "contig"),     # above 128 rows (tile kernel)
     (Q0, F32, 64, 5, 256, 2, 1, 1, 1, "kstride"),
     (QK, F16, 64, 3, 512, 1, 2, 1, 2, "kstride"),
     (Q0, F16, 200, 64, 256, 1, 1, 1, 1, "padded"),      # fp16, row stride K + 8: in place

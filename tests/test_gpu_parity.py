@@ -207,7 +207,9 @@ def test_gemm_odd_shapes(dev, qt, K):
 def test_gemm_large_m_is_sliced(dev):
     w = O.gen_weights(O.Q4_K, 64, 1024, seed=41)
     A = O.gen_act(300, 1024, seed=42)
-    check_gemm(gpu_gemm(w, A, dev), w, A, "M=300")
+    check_gemm(gpu_gemm(w, A, dev), w, A, "M=300")     # AUTO: one launch of the tile kernel
+    for algo in (bf.ALGO_MFMA, bf.ALGO_DENSE, bf.ALGO_SIMPLE):
+        check_gemm(gpu_gemm(w, A, dev, algo=algo), w, A, f"M=300 algo={algo}, slices of 128 rows")
 
 
 # ------------------------------------------------------------------ interface behaviour

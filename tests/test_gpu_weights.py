@@ -73,14 +73,15 @@ def k_columns(rng, count):
     return np.unique(ks)[:count] if np.unique(ks).size >= count else np.unique(ks)
 
 
-def readout(w, dw, ks, M, algo, dev):
-    """W_eff[:, ks] as computed by kernel `algo` at batch M (rows of A one-hot)."""
+def readout(w, dw, ks, M, algo, dev, shift=0):
+    """W_eff[:, ks] as computed by kernel `algo` at batch M (rows of A one-hot, `shift` elements into a buffer)."""
     cols = []
     for i0 in range(0, ks.size, M):
         chunk = ks[i0:i0 + M]
         A = np.zeros((M, K), np.uint16)
         A[np.arange(chunk.size), chunk] = np.float16(1.0).view(np.uint16)
-        Ad = torch.from_numpy(A.view(np.int16)).to(dev)
+        Ad = torch.zeros(M * K + shift, dtype=torch.int16, device=dev)[shift:]
+        Ad.copy_(torch.from_numpy(A.view(np.int16)).reshape(-1))
         C = torch.full((M, N), float("nan"), device=dev)
         bf.gemm(w.qtype, dw[0], dw[1], Ad, C, M, N, K, algo=algo)
         torch.cuda.synchronize()
@@ -126,6 +127,12 @@ KERNELS = {
 KERNELS[O.Q4_0_PLANES] = [k for k in KERNELS[O.Q4_0] if k[0] != bf.ALGO_SLAB]     # the slab kernel reads blocks only
 
 
+# AUTO on the tile kernel (batches above 128; its other tile shapes: tests/test_gpu_tile.py) and, with activations
+# off their 16-byte boundary, on the block-wise kernel (Q4_0 formats; the last two with activations through LDS)
+TILE = [(bf.ALGO_AUTO, M, "f16", 0) for M in (129, 256, 300, 2000)]
+BLOCK = [(bf.ALGO_AUTO, M, "f32", 1) for M in (1, 20, 40, 64, 2200, 4200)]
+
+
 @pytest.mark.parametrize("qt", [O.Q4_K, O.Q4_0, O.Q4_0_PLANES], ids=lambda q: QT_NAME[q])
 def test_kernel_weights_bitwise(dev, qt):
     w = wide_scale_weights(qt, seed=900 + qt)
@@ -140,8 +147,9 @@ def test_kernel_weights_bitwise(dev, qt):
         # the sample holds weights where one rounding of the exact value differs from the dequant
         once = single_rounding_q4k(w, ks).astype(np.float32)
         assert (once != ref["f16"]).sum() >= 3
-    for algo, M, form in KERNELS[qt]:
-        got = readout(w, (Wd, auxd), ks, M, algo, dev)
+    kernels = [(*k, 0) for k in KERNELS[qt]] + TILE + (BLOCK if qt != O.Q4_K else [])
+    for algo, M, form, shift in kernels:
+        got = readout(w, (Wd, auxd), ks, M, algo, dev, shift)
         bad = np.nonzero(got != ref[form])              # as values: +0 and -0 are one weight
         assert bad[0].size == 0, (f"{QT_NAME[qt]} algo={algo} M={M}: {bad[0].size} weights differ from the "
                                   f"{form} dequant, first at n={bad[0][0]} k={ks[bad[1][0]]}: "

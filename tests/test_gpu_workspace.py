@@ -273,7 +273,7 @@ def test_threads_interleave_two_launch_calls_on_one_stream(dev):
     overwritten by the other's between its two launches: every output equals
     the single-threaded call's bits."""
     s = new_stream()
-    N, K, M, MG = 5120, 5120, 64, 4
+    N, K, M, MG = 5120, 5120, 64, 12                   # (up to eight rows go to the GEMM kernel unstaged)
     ops = []
     for t in range(2):
         _, W, aux, _, Ad = case(O.Q4_K, N, K, M, 200 + 10 * t, dev)

@@ -29,6 +29,32 @@ def test_plans(checker, part):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
+def plan(checker, kind, *shape):
+    r = subprocess.run([checker, kind, *map(str, shape)], capture_output=True, text=True, check=True, timeout=60)
+    return tuple(map(int, r.stdout.split()))
+
+
+def test_tile_shapes_reach_every_form(checker):
+    """The GPU tests' shapes run the form each stands for, and together every tile
+    shape uncut and cut, with and without whole rounds before the cut ones."""
+    from test_gpu_tile import FORMS
+    for shape, (ta, nb, rounds, s) in FORMS.items():
+        TA, NB, F, R, S, slices = plan(checker, "tile", *shape)
+        assert (TA, NB, F // 256, S, slices) == (ta, nb, rounds, s, 0) and R, shape
+    forms = {(ta, nb, rounds > 0, s > 1) for ta, nb, rounds, s in FORMS.values()}
+    for tile in ((2, 1), (3, 1), (4, 1), (4, 2)):
+        assert {f[3] for f in forms if f[:2] == tile} == {True, False}, tile
+    assert {(3, 1, True, True), (4, 1, True, True), (4, 2, True, True), (3, 1, False, True), (4, 1, False, True)} <= forms
+
+
+def test_block_shapes_reach_every_form(checker):
+    from test_gpu_block import FORMS
+    for shape, form in FORMS.items():
+        assert plan(checker, "block", *shape) == form, shape
+    every = {(mt, nt, 8) for mt in (1, 2, 3, 4) for nt in (1, 2)} | {(mt, 0, nw) for mt in (3, 4) for nw in (4, 8)}
+    assert set(FORMS.values()) == every
+
+
 def test_fp32_rows_inside_the_gemm():
     """ggml hook: up to eight fp32 rows go to the LDS kernel itself (no
     workspace) wherever its plan keeps all of A; nine rows, and plans with an
