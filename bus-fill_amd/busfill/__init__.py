@@ -188,20 +188,30 @@ def _ptr(t) -> int | None:
     return t.data_ptr()
 
 
+def _first_current_stream() -> int:
+    """The current stream's handle; initialises torch's GPU state, then leaves
+    the lookup to the two calls torch.cuda.current_stream() makes for it (a
+    Stream object per call costs 2.8 us, these 0.2: a batch-1 call of a small
+    matrix is bound by the host, 7.5 -> 5.0 us at 1024 x 1024), but in a forked
+    child, where torch refuses the GPU."""
+    global _current_stream
+    import torch
+    handle = torch.cuda.current_stream().cuda_stream
+    names = ("_cuda_getCurrentRawStream", "_cuda_getDevice", "_cuda_isInBadFork")
+    if all(hasattr(torch._C, n) for n in names):
+        raw, device, bad_fork = (getattr(torch._C, n) for n in names)
+        _current_stream = lambda: torch.cuda.current_stream().cuda_stream if bad_fork() else raw(device())  # noqa: E731
+    else:
+        _current_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+    return handle
+
+
+_current_stream = _first_current_stream
+
+
 def _stream(stream) -> int | None:
-    """A stream's handle; None is the current stream.  Once torch's GPU state is
-    up in this process (never in a forked child, where torch refuses), its
-    handle comes from the two calls torch.cuda.current_stream() makes for it: a
-    Stream object per call costs 2.8 us, and a batch-1 call of a small matrix is
-    bound by the host (7.5 -> 5.0 us at 1024 x 1024)."""
     if stream is None:
-        import torch
-        if torch.cuda.is_initialized():
-            try:
-                return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
-            except AttributeError:               # (names of torch's own)
-                pass
-        return torch.cuda.current_stream().cuda_stream
+        return _current_stream()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
