@@ -358,8 +358,8 @@ bf_status run_gemm(bf_qtype qtype, const void* W, const void* W_aux, const uint1
 }
 
 // Workspace bytes of a call with lda = K, ldc = N and aligned operands (the
-// operands' addresses only decide between the fast kernels and the simple one,
-// which needs none).
+// operands' addresses only decide between the fast kernels and the block-wise
+// or simple one, which need none).
 size_t gemm_workspace_bytes(bf_qtype qtype, bf_otype otype, int M, int N, int K) {
     uint8_t* const fake = (uint8_t*)(uintptr_t)4096;      // aligned placeholders, never dereferenced
     if (check_gemm(qtype, fake, qtype == BF_Q4_0_PLANES ? fake : nullptr, (const uint16_t*)fake, K, fake, N, otype,
@@ -375,7 +375,8 @@ size_t gemm_workspace_bytes(bf_qtype qtype, bf_otype otype, int M, int N, int K)
 }
 
 // Scratch of bf_gemm_noalloc: the K-split and dense kernels' row-group
-// counters and partial sums, in place of the workspace bf_gemm allocates per
+// counters and partial sums and the tile kernel's (never more than a 128-row
+// dense launch's), in place of the workspace bf_gemm allocates per
 // stream (34 MiB: the dense kernel's 256 workgroups x two 128 x 128 fp32
 // pieces plus counters for up to 8192 row groups).  Each
 // GPU the library runs on holds its own copy until the process ends.  In host

@@ -25,12 +25,16 @@
 //   2048 x 16384 x 5120).
 // * LDS rows are 128 bytes (64 k); their 16-byte chunk c sits at c ^ ((row / 2)
 //   % 8), so the 32 rows of a fragment read fall on distinct banks.
-// * Bound: power.  At 2048 x 16384 x 5120 the NB = 1 kernel issues an MFMA on
-//   68 % of the SIMD cycles (1504 of a step's cycles for 1024 of MFMA) at a
-//   clock of 1.44 GHz; without its activation loads the chip clocks at 1.68
-//   GHz.  The NB = 2 tile halves that traffic per flop: 356 -> 327-340 us
-//   (1010-1050 TFLOP/s; a library fp16 product of this size takes 386-395 us
-//   on decoded weights).
+// * Bound by neither the matrix cores' rate nor the clock alone: MFMAs take
+//   57-61 % of the SIMD cycles at 1.6-1.7 GHz with NB = 2 (2048 x 16384 x 5120:
+//   328-336 us, 1020-1050 TFLOP/s) and 43-47 % at 1.9-2.0 GHz with NB = 1 (512 x
+//   16384 x 5120: 93-97 us); an 8192^3 bf16 library product reached 1211 TFLOP/s on
+//   such a chip, a library fp16 product of the first size takes 386-395 us on
+//   decoded weights.  The compiler's own waits for the weight words count the DMAs
+//   too (vmcnt(3) to vmcnt(6) once per step; planes, whose scales are copied while
+//   fresh, vmcnt(0) once per super-group): stricter than the data needs, and not
+//   yet taken out.  NB = 2 halves the operand traffic per flop of NB = 1 (2048
+//   rows: 356 -> 327-340 us).
 // * Measured (Q4_K, us per GEMM, before -> after): 17408 x 5120 at 512 / 2000
 //   rows 150-165 / 609-648 -> 108 / 355-369; 5120 x 17408 at 2000 rows
 //   572-606 -> 348-359; 5120 x 5120 at 300 / 512 rows 52-58 / 76-80 -> 35 / 43.
@@ -344,7 +348,7 @@ struct Tile {
 
 // Workgroups [0, F): whole tiles, straight to C.  Workgroups F ..: the R =
 // tiles - F remaining ones, each cut in S ranges of super-groups whose sums go
-// to the workspace ([split][tile][row][128] fp32; S > 1) for k_tile_sum.
+// to the workspace ([split][tile][row][128 NB] fp32; S > 1) for k_tile_sum.
 template <int QT, int TA, int NB>
 __global__ __launch_bounds__(kTlThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_gemm_tile(const uint8_t* W, const uint8_t* Waux, const uint16_t* A, int lda, void* C, int ldc, int out_f16,

@@ -21,7 +21,7 @@ struct TilePlan {
 
 // Microseconds of a plan, from measured launches (Q4_K): a super-group of each
 // tile shape takes `lo` up to 0.4 of the CUs busy and up to `hi` with all of
-// them (the chip is bound by power: fewer busy CUs clock higher), a round 6.5
+// them (with fewer busy CUs the chip clocks higher), a round 6.5
 // for its start and end; the cut tiles' partials are written and read once,
 // and their sum is a launch of its own.
 inline double tile_cost(int TA, int NB, int nsg, int cus, int F, int R, int S, size_t piece) {

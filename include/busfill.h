@@ -12,12 +12,13 @@
  * describes in RESULTS.md:84-96) with a host-callable function.
  *
  * Conventions
- *   - All pointers are DEVICE pointers owned by the caller.  Two kernels
+ *   - All pointers are DEVICE pointers owned by the caller.  Three kernels
  *     exchange partial sums between workgroups and need a workspace: the
  *     K-split kernel (BF_ALGO_SPLIT, which bf_gemm picks for 9-32 batch rows
- *     per launch when the activations do not fit in LDS) and the dense kernel
- *     (BF_ALGO_DENSE, above 32 rows, and from 9 or 17 rows on matrices of
- *     3 * 2^24 weights or more).  Three ways to provide it:
+ *     per launch when the activations do not fit in LDS), the dense kernel
+ *     (BF_ALGO_DENSE, at 33-128 rows, and from 9 or 17 rows on matrices of
+ *     3 * 2^24 weights or more) and the tile kernel (above 128 rows; never more
+ *     than the dense kernel at 128).  Three ways to provide it:
  *       * bf_gemm_ws / bf_gemm_batched_ws / bf_busfill_q4_ws: the caller owns
  *         it (size from bf_gemm_workspace_bytes / bf_gemm_batched_workspace_bytes);
  *         the library allocates nothing and keeps no state between calls.
@@ -135,8 +136,8 @@ bf_status bf_gemm_ex(bf_qtype qtype, const void* W, const void* W_aux,
  * hipMalloc).  No counterpart in the reference, whose kernel needs no scratch.
  * Same arguments, kernels and results as bf_gemm, bit for bit; where bf_gemm's
  * cross-workgroup exchanges (the K-split kernel at 9-32 batch rows per launch
- * when the activations do not fit in LDS, the dense kernel above 32 rows and
- * on large matrices) use
+ * when the activations do not fit in LDS, the dense kernel at 33-128 rows and
+ * on large matrices, the tile kernel above) use
  * the workspace it allocates per stream, this call uses a 34 MiB scratch
  * array in device memory that each GPU holds for the life of the process.  It
  * calls no hipMalloc or hipFree; its first call on a device looks up that
@@ -149,7 +150,8 @@ bf_status bf_gemm_ex(bf_qtype qtype, const void* W, const void* W_aux,
  * BF_ERR_INVALID, enqueueing nothing, for a shape whose launches need more
  * than 34 MiB of scratch (K-split partials of S splits x N x M rows in fp32,
  * 11 MB at the 27B-class layer's largest shapes at M = 32; dense partials of
- * 256 workgroups x 2 x 128 x M rows, 32 MiB at M = 128). */
+ * 256 workgroups x 2 x 128 x M rows, 32 MiB at M = 128, which the tile kernel's
+ * plans keep to). */
 bf_status bf_gemm_noalloc(bf_qtype qtype, const void* W, const void* W_aux,
                           const uint16_t* A, int lda, void* C, int ldc, bf_otype otype,
                           int M, int N, int K, void* stream);
@@ -200,7 +202,7 @@ typedef struct {
  * concurrently.  The GEMMs are grouped by the kernel bf_gemm would give each:
  * those on the LDS-staged kernel (batch 1-8, per batch size), those on the
  * K-split kernel (9-32 rows whose activations do not fit in LDS; 9-16 and
- * 17-32 rows apart) and those on the dense kernel (above 32 rows or from 9
+ * 17-32 rows apart) and those on the dense kernel (33-128 rows or from 9
  * rows on large matrices, per batch size) each share one launch per eight
  * GEMMs (the dense ones one sum launch too), so one GEMM's tail overlaps the next one's weight stream and
  * launch gaps go away (a decoder layer's linears); any other GEMM runs as one
