@@ -12,7 +12,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def planner(tmp_path_factory):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
@@ -24,22 +24,22 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("part", ["dequant", "block_grid", "block_choice", "tile_grid", "tile_choice"])
-def test_plans(checker, part):
-    r = subprocess.run([checker, part], capture_output=True, text=True, timeout=120)
+def test_plans(planner, part):
+    r = subprocess.run([planner, part], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
 
 
-def plan(checker, kind, *shape):
-    r = subprocess.run([checker, kind, *map(str, shape)], capture_output=True, text=True, check=True, timeout=60)
+def plan(planner, kind, *shape):
+    r = subprocess.run([planner, kind, *map(str, shape)], capture_output=True, text=True, check=True, timeout=60)
     return tuple(map(int, r.stdout.split()))
 
 
-def test_tile_shapes_reach_every_form(checker):
+def test_tile_shapes_reach_every_form(planner):
     """The GPU tests' shapes run the form each stands for, and together every tile
     shape uncut and cut, with and without whole rounds before the cut ones."""
     from test_gpu_tile import FORMS
     for shape, (ta, nb, rounds, s) in FORMS.items():
-        TA, NB, F, R, S, slices = plan(checker, "tile", *shape)
+        TA, NB, F, R, S, slices = plan(planner, "tile", *shape)
         assert (TA, NB, F // 256, S, slices) == (ta, nb, rounds, s, 0) and R, shape
     forms = {(ta, nb, rounds > 0, s > 1) for ta, nb, rounds, s in FORMS.values()}
     for tile in ((2, 1), (3, 1), (4, 1), (4, 2)):
@@ -47,10 +47,10 @@ def test_tile_shapes_reach_every_form(checker):
     assert {(3, 1, True, True), (4, 1, True, True), (4, 2, True, True), (3, 1, False, True), (4, 1, False, True)} <= forms
 
 
-def test_block_shapes_reach_every_form(checker):
+def test_block_shapes_reach_every_form(planner):
     from test_gpu_block import FORMS
     for shape, form in FORMS.items():
-        assert plan(checker, "block", *shape) == form, shape
+        assert plan(planner, "block", *shape) == form, shape
     every = {(mt, nt, 8) for mt in (1, 2, 3, 4) for nt in (1, 2)} | {(mt, 0, nw) for mt in (3, 4) for nw in (4, 8)}
     assert set(FORMS.values()) == every
 
